@@ -2,7 +2,7 @@
 
     python -m fft_amd.build [--incremental]       (or fft_amd.build.build())
 
-The four translation units compile in parallel; the FP32 and FP64 pass-kernel
+The translation units compile in parallel; the FP32 and FP64 pass-kernel
 instantiations dominate the build time.
 """
 from __future__ import annotations
@@ -16,7 +16,8 @@ PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG, "csrc")
 OBJ = os.path.join(PKG, "_obj")
 LIB = os.path.join(PKG, "libafft_mi355x.so")
-SOURCES = ["afft_kernels_f32.hip", "afft_kernels_f64.hip", "afft_aux.hip", "afft_plan.hip", "afft_queue.hip", "afft_mfma.hip",
+SOURCES = ["afft_kernels_f32_cols.hip", "afft_kernels_f32.hip", "afft_kernels_f32_realcols.hip", "afft_kernels_f64_cols.hip",
+           "afft_kernels_f64.hip", "afft_kernels_f64_realcols.hip", "afft_aux.hip", "afft_plan.hip", "afft_queue.hip", "afft_mfma.hip",
            "afft_realpair.hip", "afft_fused.hip", "afft_real4.hip", "afft_tiny.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -1,6 +1,10 @@
-// FP32 instantiations of the pass kernels.
+// FP32 instantiations of the pass kernels (row passes here; the _cols and
+// _realcols units include this file for their part).
 // Column tiles: 16 columns (128-byte segments) up to L = 1024; beyond that the
 // 160 KiB LDS of a CU bounds CT * L.
+#ifndef AFGPU_PART
+#define AFGPU_PART 0
+#endif
 #define AFGPU_T float
 #define AFGPU_ROW_MAX 16384
 #define AFGPU_ROW_HX_MAX 32768

@@ -1,0 +1,3 @@
+// FP32 column passes with a real pass.
+#define AFGPU_PART 2
+#include "afft_kernels_f32.hip"

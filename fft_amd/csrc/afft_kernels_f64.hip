@@ -1,6 +1,9 @@
 // FP64 instantiations of the pass kernels (16-byte elements halve what fits
 // in LDS, so tiles are half the FP32 ones and rows stop at 8192, 16384 with
 // half-LDS tiles).
+#ifndef AFGPU_PART
+#define AFGPU_PART 0
+#endif
 #define AFGPU_T double
 #define AFGPU_ROW_MAX 8192
 #define AFGPU_ROW_HX_MAX 16384

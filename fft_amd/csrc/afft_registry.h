@@ -20,6 +20,27 @@ struct PassVariant {
   PassLaunchFn<T> launch;
 };
 
+// The compiled variants of one part (afft_variants.inc).
+template <typename T>
+struct PassList {
+  const PassVariant<T>* v;
+  int n;
+};
+template <typename T, int PART>
+PassList<T> pass_part();
+template <>
+PassList<float> pass_part<float, 0>();
+template <>
+PassList<float> pass_part<float, 1>();
+template <>
+PassList<float> pass_part<float, 2>();
+template <>
+PassList<double> pass_part<double, 0>();
+template <>
+PassList<double> pass_part<double, 1>();
+template <>
+PassList<double> pass_part<double, 2>();
+
 // Looks up the compiled variant; returns nullptr when none exists.
 template <typename T>
 const PassVariant<T>* find_pass(int L, int CT, int colmap, int epi, int store_t, int sv = 0, int hx = 0);
