@@ -21,14 +21,15 @@ __device__ __forceinline__ void wexp(idx_t e, idx_t M, double& c, double& s) {
 template <typename T>
 __global__ void gen_stage_tw_kernel(cx<T>* out, StageList sl) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= sl.total) return;
+  if (i >= 2 * sl.total) return;
+  const bool by_r = i >= sl.total;  // the second copy, [r - 1][k]
   // stage 0 (Ns = 1) multiplies by nothing and has no entries
   for (int s = 1; s < sl.nstage; s++) {
-    int beg = sl.off[s], cnt = sl.ns[s] * (sl.radix[s] - 1);
+    int beg = sl.off[s] + (by_r ? sl.total : 0), cnt = sl.ns[s] * (sl.radix[s] - 1);
     if (i >= beg && i < beg + cnt) {
       int rel = i - beg;
-      int k = rel / (sl.radix[s] - 1);
-      int r = rel % (sl.radix[s] - 1) + 1;
+      int k = by_r ? rel % sl.ns[s] : rel / (sl.radix[s] - 1);
+      int r = (by_r ? rel / sl.ns[s] : rel % (sl.radix[s] - 1)) + 1;
       double c, sn;
       wexp((idx_t)r * k, (idx_t)sl.ns[s] * sl.radix[s], c, sn);
       out[i] = cx<T>{(T)c, (T)sn};
@@ -68,7 +69,7 @@ __global__ void gen_real_tw_kernel(cx<T>* out, idx_t L) {
 template <typename T>
 hipError_t gen_stage_tw(cx<T>* out, const StageList& sl, hipStream_t st) {
   if (sl.total == 0) return hipSuccess;
-  hipLaunchKernelGGL(gen_stage_tw_kernel<T>, dim3((sl.total + 255) / 256), dim3(256), 0, st, out, sl);
+  hipLaunchKernelGGL(gen_stage_tw_kernel<T>, dim3((2 * sl.total + 255) / 256), dim3(256), 0, st, out, sl);
   return hipGetLastError();
 }
 template <typename T>

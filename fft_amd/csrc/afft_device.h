@@ -266,7 +266,8 @@ struct StageNs<L, SV, 0> {
 
 // Offset (in complex entries) of stage S's twiddles in the per-length stage
 // table.  Stage S (S >= 1) has Ns * (R - 1) entries laid out [k][r - 1] with
-// value W_{Ns*R}^{r*k}.
+// value W_{Ns*R}^{r*k}.  A second copy of all stages, at the offset past the
+// last one, lays each out [r - 1][k].
 template <int L, int SV, int S>
 struct StageTwOff {
   static constexpr int value = StageTwOff<L, SV, S - 1>::value +

@@ -194,11 +194,30 @@ __device__ __forceinline__ void run_stages(Regs<T, L, SV>& v, int t, LdsAt& lat,
     if constexpr (NS > 1) {
       const int j = t + b * TPT;
       const int k = j & (NS - 1);
-      const cx<T>* tp = tw + StageTwOff<L, SV, S>::value + k * (R - 1);
-      static_for<R - 1>([&](auto rc) AFGPU_INLINE {
-        constexpr int r = decltype(rc)::value + 1;
-        a[r] = cmul(a[r], tp[r - 1]);
-      });
+      if constexpr (ST == 1 && L >= 4096) {
+        // row-mapped: consecutive lanes hold consecutive k, so in the table's
+        // second copy, laid out [r - 1][k], each load covers whole lines; in
+        // [k][r - 1] a 16-byte load touches a line per lane, and the last
+        // stage of a long row (254 KB of twiddles for 32768 points) kept the
+        // CU's cache path busier than the data did.  512 MiB moved per
+        // direction: 32768 x 1024 177 -> 156 us, FP64 16384 x 1024 138 -> 125,
+        // 16384 x 2048 139 -> 137, r2c 16384 146 -> 140; rows of 64..2048
+        // points, whose tables stay in the L1, lose 3-4 % to the larger number
+        // of loads (1024 x 30011 174 -> 181) and keep the first copy
+        const cx<T>* tp = tw + StageTwOff<L, SV, Sched<L, SV>::NST>::value + StageTwOff<L, SV, S>::value + k;
+        static_for<R - 1>([&](auto rc) AFGPU_INLINE {
+          constexpr int r = decltype(rc)::value + 1;
+          a[r] = cmul(a[r], tp[(r - 1) * NS]);
+        });
+      } else {
+        // column-mapped: the lanes of a column tile share k, whose R - 1
+        // entries are contiguous
+        const cx<T>* tp = tw + StageTwOff<L, SV, S>::value + k * (R - 1);
+        static_for<R - 1>([&](auto rc) AFGPU_INLINE {
+          constexpr int r = decltype(rc)::value + 1;
+          a[r] = cmul(a[r], tp[r - 1]);
+        });
+      }
     }
     Dft<T, R>::run(a);
     static_for<R>([&](auto rc) AFGPU_INLINE { v[b + decltype(rc)::value * NB] = a[decltype(rc)::value]; });

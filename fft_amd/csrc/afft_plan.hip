@@ -332,7 +332,7 @@ const void* get_table(int type, idx_t n, int bits) {
       if (s >= 1) off += ns[s] * (radix[s] - 1);
     }
     sl.total = off;
-    size_t bytes = sizeof(cx<T>) * (size_t)(off > 0 ? off : 1);
+    size_t bytes = sizeof(cx<T>) * (size_t)(off > 0 ? 2 * off : 1);  // [k][r - 1] and [r - 1][k]
     e = hipMalloc(&p, bytes);
     if (e == hipSuccess) e = gen_stage_tw<T>((cx<T>*)p, sl, nullptr);
   } else if (type == 3) {  // A operands of the MFMA DFT-256 tile (bits: 1 = BF16 three-way)
