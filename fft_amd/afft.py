@@ -11,6 +11,7 @@ stream-aware extension (include/afft_gpu.h)."""
 from __future__ import annotations
 
 import ctypes
+import sys
 
 import numpy as np
 
@@ -39,6 +40,25 @@ def required_counts(kind: str, dims, fmt: int, batch: int = 1):
     if kind == "r":
         return (n * b, 2 * m * b, 0) if il else (n * b, m * b, m * b)
     return (2 * m * b, 0, n * b) if il else (m * b, m * b, n * b)
+
+
+def _torch_dtype(dtype):
+    """torch's name of a numpy element type, None while torch is not loaded."""
+    t = sys.modules.get("torch")
+    return None if t is None else {"float32": t.float32, "float64": t.float64}[np.dtype(dtype).name]
+
+
+def addresses(bufs, counts, dtype, tdtype):
+    """The device addresses of `bufs` after check_buffers' checks.  Buffers that
+    are plainly fine (the usual call) are recognised without building names or
+    messages (a 4096-point call: 28.4 -> 18.6 us)."""
+    for x, need in zip(bufs, counts):
+        if need and not (type(x) is int and x) and not (
+                tdtype is not None and getattr(x, "dtype", None) is tdtype and x.is_cuda and x.is_contiguous()
+                and x.numel() >= need):
+            check_buffers(bufs, counts, dtype)
+            break
+    return [x.data_ptr() if hasattr(x, "data_ptr") else _lib.ptr(x) for x in bufs]
 
 
 def check_buffers(bufs, counts, dtype):
@@ -100,6 +120,9 @@ class _Transform:
         self._mem = ctypes.create_string_buffer(size)
         st = getattr(L, f"afft_{p}_{self._kind}_create")(nd, arr, self.format, self._mem, int(impl))
         self.state = st if st else None
+        if self.state:
+            self._counts = required_counts(self._kind, self.dims, self.format)
+            self._tdtype = _torch_dtype(self.dtype)
 
     def __bool__(self):
         return self.state is not None
@@ -133,8 +156,7 @@ class complex_transform(_Transform):
 
     def __call__(self, src_re, src_im, dst_re, dst_im):
         self._check()
-        check_buffers((src_re, src_im, dst_re, dst_im), required_counts(self._kind, self.dims, self.format), self.dtype)
-        self._fn_transform(self.state, _lib.ptr(src_re), _lib.ptr(src_im), _lib.ptr(dst_re), _lib.ptr(dst_im))
+        self._fn_transform(self.state, *addresses((src_re, src_im, dst_re, dst_im), self._counts, self.dtype, self._tdtype))
 
 
 class inverse_complex_transform(_Transform):
@@ -143,8 +165,7 @@ class inverse_complex_transform(_Transform):
 
     def __call__(self, src_re, src_im, dst_re, dst_im):
         self._check()
-        check_buffers((src_re, src_im, dst_re, dst_im), required_counts(self._kind, self.dims, self.format), self.dtype)
-        self._fn_transform(self.state, _lib.ptr(src_re), _lib.ptr(src_im), _lib.ptr(dst_re), _lib.ptr(dst_im))
+        self._fn_transform(self.state, *addresses((src_re, src_im, dst_re, dst_im), self._counts, self.dtype, self._tdtype))
 
 
 class real_transform(_Transform):
@@ -153,8 +174,7 @@ class real_transform(_Transform):
 
     def __call__(self, src, dst_re, dst_im):
         self._check()
-        check_buffers((src, dst_re, dst_im), required_counts("r", self.dims, self.format), self.dtype)
-        self._fn_transform(self.state, _lib.ptr(src), _lib.ptr(dst_re), _lib.ptr(dst_im))
+        self._fn_transform(self.state, *addresses((src, dst_re, dst_im), self._counts, self.dtype, self._tdtype))
 
 
 class inverse_real_transform(_Transform):
@@ -163,8 +183,7 @@ class inverse_real_transform(_Transform):
 
     def __call__(self, src_re, src_im, dst):
         self._check()
-        check_buffers((src_re, src_im, dst), required_counts("ri", self.dims, self.format), self.dtype)
-        self._fn_transform(self.state, _lib.ptr(src_re), _lib.ptr(src_im), _lib.ptr(dst))
+        self._fn_transform(self.state, *addresses((src_re, src_im, dst), self._counts, self.dtype, self._tdtype))
 
 
 def supported(impl: int) -> bool:
@@ -211,29 +230,25 @@ class Plan:
         if not st:
             raise RuntimeError(f"plan creation failed: {_lib.last_error()}")
         self.state = st
+        self._execute = L.afft_gpu_execute
+        cnt = required_counts(kind, self.dims, self.format, self.batch)
+        # by execute's (src_re, src_im, dst_re, dst_im): a real input has no
+        # src_im, a real output no dst_im
+        self._counts = cnt if len(cnt) == 4 else (cnt[0], 0) + cnt[1:] if kind == "r" else cnt + (0,)
+        self._tdtype = _torch_dtype(self.dtype)
 
     def _bufs(self, src_re, src_im, dst_re, dst_im):
-        """Checks the buffers against the plan; the real kinds use the first
-        three of the four arguments as (src, dst_re, dst_im) / (src_re, src_im,
-        dst)."""
+        """Checks the buffers against the plan and returns their addresses; the
+        real kinds use the first three of the four arguments as (src, dst_re,
+        dst_im) / (src_re, src_im, dst)."""
         if not self.state:
             raise RuntimeError("plan is closed")
-        cnt = required_counts(self.kind, self.dims, self.format, self.batch)
-        if len(cnt) == 3:
-            if self.kind == "r":
-                # execute's (src_re, src_im, dst_re, dst_im) with src_im unused
-                check_buffers((src_re, dst_re, dst_im), cnt, self.dtype)
-            else:
-                check_buffers((src_re, src_im, dst_re), cnt, self.dtype)
-        else:
-            check_buffers((src_re, src_im, dst_re, dst_im), cnt, self.dtype)
+        return addresses((src_re, src_im, dst_re, dst_im), self._counts, self.dtype, self._tdtype)
 
     def __call__(self, src_re, src_im, dst_re, dst_im, stream=None):
-        self._bufs(src_re, src_im, dst_re, dst_im)
+        a = self._bufs(src_re, src_im, dst_re, dst_im)
         h = getattr(stream, "cuda_stream", stream)
-        r = _lib.lib().afft_gpu_execute(self.state, _lib.ptr(src_re), _lib.ptr(src_im), _lib.ptr(dst_re),
-                                        _lib.ptr(dst_im), h)
-        if r != 0:
+        if self._execute(self.state, *a, h) != 0:
             raise RuntimeError(_lib.last_error())
 
     def run_range(self, first, last, src_re, src_im, dst_re, dst_im, stream=None):

@@ -61,3 +61,15 @@ def test_check_buffers_accepts_and_rejects():
     with pytest.raises(ValueError, match="second"):
         afft.check_buffers((_FakeDev(64), None, _FakeDev(64), _FakeDev(64)), cs, np.float32)
     afft.check_buffers((_FakeDev(64), _FakeDev(64), _FakeDev(64), _FakeDev(64)), cs, np.float32)
+
+
+@pytest.mark.parametrize("bad", [(127, {}), (128, {"dtype": torch.float64}), (128, {"contiguous": False})])
+def test_addresses_check_every_call(bad):
+    cnt = afft.required_counts("c", (64,), IL, 1)
+    t = afft._torch_dtype(np.float32)
+    assert afft.addresses((_FakeDev(128), None, 0x3000, None), cnt, np.float32, t) == [0x1000, None, 0x3000, None]
+    # without torch the general checks decide
+    assert afft.addresses((_FakeDev(128), None, 0x3000, None), cnt, np.float32, None) == [0x1000, None, 0x3000, None]
+    for x in (_FakeDev(bad[0], **bad[1]), None, 0, torch.zeros(128)):
+        with pytest.raises(ValueError):
+            afft.addresses((_FakeDev(128), None, x, None), cnt, np.float32, t)
