@@ -333,7 +333,7 @@ class Job(ctypes.Structure):
 
 
 class Queue:
-    """Uneven batch of 1-D FP32 transforms run in one persistent launch
+    """Uneven batch of 1-D FP32 transforms run in persistent launches
     (afft_gpu_queue_*)."""
 
     def __init__(self, max_jobs: int, max_log2n: int = 16):

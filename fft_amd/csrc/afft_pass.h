@@ -429,8 +429,10 @@ __device__ __forceinline__ void fft_tile(const PassParams<T>& p, int tile, int t
       ib = 0;
       ob = 0;
       if (active) {
-        in_re = reinterpret_cast<const T*>(p.col_ptrs[2 * col]);
-        out_re = reinterpret_cast<T*>(p.col_ptrs[2 * col + 1]);
+        // (cast through the global address space: a pointer read from memory
+        // would be accessed with flat instructions)
+        in_re = (const T*)(__attribute__((address_space(1))) const T*)p.col_ptrs[2 * col];
+        out_re = (T*)(__attribute__((address_space(1))) T*)p.col_ptrs[2 * col + 1];
       }
     }
   }

@@ -2551,6 +2551,7 @@ int stage_list(int L, int sv, int* radix, int* ns) {
       case 512: return fill_stages<512, 1>(radix, ns);
       case 1024: return fill_stages<1024, 1>(radix, ns);
       case 2048: return fill_stages<2048, 1>(radix, ns);
+      case 16384: return fill_stages<16384, 1>(radix, ns);
       default: return 0;
     }
   }

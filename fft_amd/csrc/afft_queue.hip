@@ -1,5 +1,6 @@
 // afft_queue.hip -- thousands of 1-D FP32 transforms of uneven power-of-two
-// sizes, kinds and directions in ONE persistent launch.
+// sizes, kinds and directions in one call: the task lists and the persistent
+// kernel of the short jobs (and of few long ones).
 //
 // There is no counterpart in afft (one plan per shape, one call per
 // transform); the individual transforms computed are exactly afft's c / ci /
@@ -10,8 +11,10 @@
 //     complex length L <= 4096 (c2c n <= 4096, real n <= 8192); the tile runs
 //     them side by side exactly like a row pass, each column with its own
 //     src / dst (PassParams::col_ptrs);
-//   - a longer job (complex length m = 8192 .. 65536) becomes a chain of tile
-//     tasks over its own scratch slot: [real pre-pass tiles (c2r)] -> four-step
+//   - longer jobs (complex length m = 8192 .. 65536), where they are enough to
+//     fill the GPU, run as whole rows and pass pairs in launches of their own
+//     (afft_queue_long.hip);
+//   - otherwise such a job becomes a chain of tile tasks over its own scratch slot: [real pre-pass tiles (c2r)] -> four-step
 //     pass-A tiles (m/256-point columns, 16..64 columns each, W_m twiddle) ->
 //     pass-B tiles (16 rows of 256 points, columns-fastest store) -> [real
 //     post-pass tiles (r2c)].  Every tile of one step can run on a different
@@ -37,7 +40,7 @@
 // polls the counter with atomics (performed in the L2) and then invalidates
 // its CU's L1 (buffer_inv sc0); no L2-wide write-back or invalidation is
 // needed.  afft_gpu_queue_launch issues only kernels (a
-// reset kernel for the counters and the persistent kernel), so it can be
+// reset kernel for the counters and the persistent kernels), so it can be
 // captured in a HIP graph and replayed.
 #include <hip/hip_runtime.h>
 
@@ -52,55 +55,25 @@
 #include "../../include/afft_gpu.h"
 #include "afft_aux.h"
 #include "afft_pass.h"
+#include "afft_queue_tasks.h"
 
 namespace afgpu {
 
 const void* queue_table(int type, idx_t n, int bits);  // afft_plan.hip (twiddle cache)
 void queue_set_err(const char* msg);
 
-enum { QT_GROUP = 0, QT_RPRE = 1, QT_BIGA = 2, QT_BIGB = 3, QT_RPOST = 4 };
 constexpr int kQThreads = 256;
-constexpr int kQMaxLog2 = 16;
 constexpr int kBigN2 = 256;
 constexpr int kRealTile = 2048;  // bin pairs per real-pass tile
 constexpr int kLag = 128;        // default jobs between consecutive steps of one chain (per XCD list)
-constexpr int kXcd = 8;          // XCDs of an MI355X: one chain list each
-constexpr int kCtr = 16;         // ints between counters (one 64-byte line each)
-
-struct QTask {
-  int type;
-  int lg;     // log2 of the complex length (group: L, chain: m)
-  int kind;   // afft_gpu_c / ci / r / ri
-  int count;  // group: jobs; chain: index of this step within the job
-  int first;  // first (src, dst) pair in the pointer table; a chain's scratch follows
-  int job;    // chain: job index (dependency counters)
-  int tile;   // chain: tile index within the step
-  int need;   // chain: tiles of the previous step to wait for (0: none)
-};
-
-struct QTables {
-  const cx<float>* stage[kQMaxLog2 + 1];  // stage twiddles of an L-point tile, by log2 L
-  const cx<float>* tw4[kQMaxLog2 + 1];    // four-step hi table (lo follows), by log2 m
-  const cx<float>* real[kQMaxLog2 + 1];   // W_{2L}^k, by log2 L
-};
-
-// Written by prepare, read by every launch: a launch (or a replay of a captured
-// one) runs the task list of the latest prepare.
-struct QListHdr {
-  int list_off[kXcd + 2];  // kXcd chain lists, then the group list, then the end
-  int ndeps;               // step counters to clear (4 per chain job)
-};
-
-struct QArgs {
-  const QTask* tasks;  // kXcd chain lists, then the shared group list
-  const unsigned long long* ptrs;
-  int* counter;        // list l pops through counter[l * kCtr]
-  const QListHdr* hdr;
-  int* deps;       // 4 step counters per chain job
-  int* status;     // set to 1 when a dependency wait hits the spin limit
-  long long spin_limit;
-  const QTables* tab;  // device copy: indexed by log2 length at run time
-};
+// Long jobs (2^13 complex points and more) run as whole rows and pass pairs
+// (afft_queue_long.hip) from this many complex points of them in all, as chains
+// below.  Chains against rows and pairs, in us: 100 jobs of 2^13..2^15 (1.9 M
+// points) 46 / 85, 300 (5.6 M) 69 / 91, 700 of 2^6..2^16 (6.5 M) 94 / 115,
+// 1000 (9.3 M) 120 / 124, 500 of 2^13..2^15 (9.4 M) 110 / 98, 1000 (19 M)
+// 190 / 124, 300 of 2^16 (17 M) 179 / 129, 3000 of 2^6..2^16 (28 M) 295 / 246.
+constexpr size_t kLongPoints = (size_t)10 << 20;
+constexpr int kStatus = kQLists;  // counter slot of the status flag
 
 template <int L>
 struct QGroupCT {
@@ -121,9 +94,9 @@ __device__ __noinline__ void q_group(const QArgs& a, const QTask& tk, int tid, c
   p.n_blo = 1;
   p.in_il = 1;
   p.out_il = 1;
-  p.col_ptrs = a.ptrs + 2 * (idx_t)tk.first;
-  p.stage_tw = a.tab->stage[tk.lg];
-  p.real_tw = a.tab->real[tk.lg];
+  p.col_ptrs = q_global(a.ptrs) + 2 * (idx_t)tk.first;
+  p.stage_tw = q_global(q_const(a.tab)->stage[tk.lg]);
+  p.real_tw = q_global(q_const(a.tab)->real[tk.lg]);
   if (tk.kind == afft_gpu_c || tk.kind == afft_gpu_ci) {
     p.swap_in = p.swap_out = tk.kind == afft_gpu_ci;
     fft_tile<float, L, CT, false, EPI_PLAIN, false>(p, 0, tid, lds);
@@ -194,7 +167,7 @@ int q_chain_a_tiles(int lg) {
 // (m complex); c2r runs the real pre-pass from src into dst and the c2c from
 // dst; r2c runs the real post-pass in place on dst.
 __device__ __noinline__ void q_chain(const QArgs& a, const QTask& tk, int tid, cx<float>* lds) {
-  int* dep = a.deps + 4 * (idx_t)tk.job;
+  int* dep = q_global(a.deps) + 4 * (idx_t)tk.job;
   if (tk.need > 0) {
     if (tid == 0) {
       long long it = 0;
@@ -214,14 +187,14 @@ __device__ __noinline__ void q_chain(const QArgs& a, const QTask& tk, int tid, c
   }
   const idx_t m = idx_t(1) << tk.lg;
   const int n1 = (int)(m / kBigN2);
-  const unsigned long long* pp = a.ptrs + 2 * (idx_t)tk.first;
-  const cx<float>* src = reinterpret_cast<const cx<float>*>(pp[0]);
-  cx<float>* dst = reinterpret_cast<cx<float>*>(pp[1]);
-  cx<float>* scr = reinterpret_cast<cx<float>*>(pp[2]);
+  const QConst<unsigned long long> pp = q_const(a.ptrs) + 2 * (idx_t)tk.first;
+  const cx<float>* src = q_global<const cx<float>>(pp[0]);
+  cx<float>* dst = q_global<cx<float>>(pp[1]);
+  cx<float>* scr = q_global<cx<float>>(pp[2]);
   const bool swap = tk.kind == afft_gpu_ci || tk.kind == afft_gpu_ri;
   if (tk.type == QT_RPRE || tk.type == QT_RPOST) {
     const bool inv = tk.type == QT_RPRE;
-    q_real_pass(inv ? src : dst, dst, m, inv, a.tab->real[tk.lg], tid, (idx_t)tk.tile * kRealTile,
+    q_real_pass(inv ? src : dst, dst, m, inv, q_global(q_const(a.tab)->real[tk.lg]), tid, (idx_t)tk.tile * kRealTile,
                 (idx_t)(tk.tile + 1) * kRealTile);
   } else if (tk.type == QT_BIGA) {
     // pass A: n1-point columns (stride 256) with the W_m twiddle, into scratch
@@ -236,12 +209,12 @@ __device__ __noinline__ void q_chain(const QArgs& a, const QTask& tk, int tid, c
     pa.n_blo = 1;
     pa.in_il = pa.out_il = 1;
     pa.swap_in = swap;
-    pa.tw4_hi = a.tab->tw4[tk.lg];
-    pa.tw4_lo = a.tab->tw4[tk.lg] + (m >> ((tk.lg + 1) / 2));
+    pa.tw4_hi = q_global(q_const(a.tab)->tw4[tk.lg]);
+    pa.tw4_lo = pa.tw4_hi + (m >> ((tk.lg + 1) / 2));
     pa.tw4_lo_bits = (tk.lg + 1) / 2;
     pa.tw4_log2n = tk.lg;  // the twiddle is computed, not read from the tables
     pa.tw4_col_shift = 0;
-    pa.stage_tw = a.tab->stage[tk.lg - 8];
+    pa.stage_tw = q_global(q_const(a.tab)->stage[tk.lg - 8]);
     switch (n1) {
       case 32: q_pass_a_tile<32>(pa, tk.tile, tid, lds); break;
       case 64: q_pass_a_tile<64>(pa, tk.tile, tid, lds); break;
@@ -261,7 +234,7 @@ __device__ __noinline__ void q_chain(const QArgs& a, const QTask& tk, int tid, c
     pb.n_blo = 1;
     pb.in_il = pb.out_il = 1;
     pb.swap_out = swap;
-    pb.stage_tw = a.tab->stage[8];
+    pb.stage_tw = q_global(q_const(a.tab)->stage[8]);
     pb.col_tiles = n1 / 16;
     fft_tile<float, kBigN2, 16, false, EPI_PLAIN, true>(pb, tk.tile, tid, lds);
   }
@@ -305,7 +278,7 @@ __global__ void __launch_bounds__(kQThreads, GROUPS) queue_kernel(QArgs a) {
   __shared__ int s_task;
   const int tid = threadIdx.x;
   // this XCD's chain list first, then the shared group list
-  const int lists[2] = {xcc_id(), kXcd};
+  const int lists[2] = {xcc_id(), QL_GROUP};
   for (int li = 0; li < 2; li++) {
     const int l = lists[li];
     const int off = a.hdr->list_off[l];
@@ -330,7 +303,7 @@ __global__ void __launch_bounds__(kQThreads, GROUPS) queue_kernel(QArgs a) {
 // kernel, not a memset, so a captured graph replays it reliably).
 __global__ void queue_reset_kernel(int* counter, int* status, int* deps, const QListHdr* hdr) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i <= kXcd) counter[i * kCtr] = 0;
+  if (i < kQLists) counter[i * kCtr] = 0;
   if (i == 0) *status = 0;
   const int ndeps = hdr->ndeps;
   for (int k = i; k < ndeps; k += gridDim.x * blockDim.x) deps[k] = 0;
@@ -389,7 +362,7 @@ struct Queue {
   size_t cap_tasks = 0;
   unsigned long long* d_ptrs = nullptr;
   size_t cap_ptrs = 0;
-  int* d_counter = nullptr;  // list counters at [l * kCtr], l = 0..kXcd; status at [(kXcd + 1) * kCtr]
+  int* d_counter = nullptr;  // list counters at [l * kCtr], l < kQLists; status at [kStatus * kCtr]
   QListHdr hdr{};
   QListHdr* d_hdr = nullptr;
   int* d_deps = nullptr;
@@ -476,7 +449,7 @@ afft_gpu_queue* afft_gpu_queue_create(size_t max_jobs, int max_log2n, void* mem)
     const int rt = (int)((((size_t)1 << lgm) / 2 + 1 + kRealTile - 1) / kRealTile);
     max_chain_tasks = std::max(max_chain_tasks, rt + q_chain_a_tiles(lgm) + (1 << (lgm - 8)) / 16);
   }
-  hipError_t e = hipMalloc(&q->d_counter, sizeof(int) * kCtr * (kXcd + 2));
+  hipError_t e = hipMalloc(&q->d_counter, sizeof(int) * kCtr * (kQLists + 1));
   if (e == hipSuccess) e = hipMalloc(&q->d_hdr, sizeof(QListHdr));
   if (e == hipSuccess) e = hipMemset(q->d_hdr, 0, sizeof(QListHdr));
   if (e == hipSuccess) e = q_reserve(q->d_tasks, q->cap_tasks, max_jobs * (size_t)max_chain_tasks);
@@ -501,7 +474,9 @@ afft_gpu_queue* afft_gpu_queue_create(size_t max_jobs, int max_log2n, void* mem)
     int bits = (lg + 1) / 2;
     q->tab.tw4[lg] = (const cx<float>*)queue_table(1, idx_t(1) << lg, bits);
     q->tab.real[lg] = (const cx<float>*)queue_table(2, idx_t(1) << lg, 0);
-    if (!q->tab.tw4[lg] || !q->tab.real[lg]) {
+    // whole rows of 2^13..2^15 points (2^14: the radix-32 schedule)
+    if (lg <= 15) q->tab.stage[lg] = (const cx<float>*)queue_table(0, idx_t(1) << lg, lg == 14);
+    if (!q->tab.tw4[lg] || !q->tab.real[lg] || (lg <= 15 && !q->tab.stage[lg])) {
       free_queue(q);
       return nullptr;
     }
@@ -535,7 +510,7 @@ int afft_gpu_queue_prepare(afft_gpu_queue* qh, const afft_gpu_job* jobs, size_t 
   }
   // bucket by (kind, complex length)
   std::vector<std::vector<size_t>> small((size_t)4 * 13);
-  std::vector<size_t> big;
+  std::vector<size_t> big, rows, pairs;
   for (size_t i = 0; i < njobs; i++) {
     const afft_gpu_job& j = jobs[i];
     const bool real = j.kind == afft_gpu_r || j.kind == afft_gpu_ri;
@@ -546,8 +521,19 @@ int afft_gpu_queue_prepare(afft_gpu_queue* qh, const afft_gpu_job* jobs, size_t 
     const int lgm = real ? j.log2n - 1 : j.log2n;
     if (lgm <= 12)
       small[(size_t)j.kind * 13 + lgm].push_back(i);
+    else if (lgm < 16)
+      rows.push_back(i);
     else
-      big.push_back(i);
+      pairs.push_back(i);
+  }
+  // few long jobs run as chains, whose tiles spread one job over many CUs
+  size_t points = 0;
+  for (size_t i : rows) points += (size_t)1 << (jobs[i].log2n - (jobs[i].kind >= afft_gpu_r ? 1 : 0));
+  points += pairs.size() << 16;
+  if (points < kLongPoints) {
+    big.swap(rows);
+    big.insert(big.end(), pairs.begin(), pairs.end());
+    pairs.clear();
   }
   q->h_tasks.clear();
   q->h_ptrs.clear();
@@ -573,11 +559,14 @@ int afft_gpu_queue_prepare(afft_gpu_queue* qh, const afft_gpu_job* jobs, size_t 
     scratch_off[c] = scratch_elems;
     scratch_elems += (size_t)1 << lgm;
   }
+  const size_t pair_off = scratch_elems;
+  scratch_elems += pairs.size() << 16;
   hipError_t e0 = q_reserve(q->d_scratch, q->cap_scratch, std::max<size_t>(scratch_elems, 1));
   if (e0 != hipSuccess) {
     queue_set_err(hipGetErrorString(e0));
     return -1;
   }
+  q->hdr.pair_scratch = q->d_scratch + pair_off;
   std::vector<int> first(big.size());
   for (size_t c = 0; c < big.size(); c++) {
     const afft_gpu_job& j = jobs[big[c]];
@@ -626,7 +615,7 @@ int afft_gpu_queue_prepare(afft_gpu_queue* qh, const afft_gpu_job* jobs, size_t 
         }
       }
   }
-  q->hdr.list_off[kXcd] = (int)q->h_tasks.size();
+  q->hdr.list_off[QL_GROUP] = (int)q->h_tasks.size();
   q->nchain = (int)nb;
   for (int lgm = 12; lgm >= 0; lgm--)
     for (int kind = 0; kind < 4; kind++) {
@@ -646,8 +635,28 @@ int afft_gpu_queue_prepare(afft_gpu_queue* qh, const afft_gpu_job* jobs, size_t 
         q->h_tasks.push_back(t);
       }
     }
+  // whole rows, longest first; pass pairs with their scratch
+  auto long_tasks = [&](int list, int type, int lo, int hi, const std::vector<size_t>& js) {
+    q->hdr.list_off[list] = (int)q->h_tasks.size();
+    for (int lg = hi; lg >= lo; lg--)
+      for (size_t i = 0; i < js.size(); i++) {
+        const afft_gpu_job& j = jobs[js[i]];
+        if (j.log2n - (j.kind >= afft_gpu_r ? 1 : 0) != lg) continue;
+        QTask t{};
+        t.type = type;
+        t.kind = j.kind;
+        t.lg = lg;
+        t.count = 1;
+        t.src = j.src;
+        t.dst = j.dst;
+        q->h_tasks.push_back(t);
+      }
+  };
+  long_tasks(QL_ROW15, QT_ROW, 15, 15, rows);
+  long_tasks(QL_ROW14, QT_ROW, 13, 14, rows);
+  long_tasks(QL_PAIR, QT_PAIR, 16, 16, pairs);
   q->ntasks = (int)q->h_tasks.size();
-  q->hdr.list_off[kXcd + 1] = q->ntasks;
+  q->hdr.list_off[kQLists] = q->ntasks;
   q->hdr.ndeps = 4 * q->nchain;
   if (q->h_tasks.size() > q->cap_tasks || q->h_ptrs.size() > q->cap_ptrs || (size_t)q->hdr.ndeps > q->cap_deps) {
     queue_set_err("queue: internal: task list exceeds the arrays sized at create");
@@ -678,31 +687,45 @@ int afft_gpu_queue_launch(afft_gpu_queue* qh, void* stream) {
   static_assert(kQLds * 4 <= 160 * 1024, "four groups per CU must fit the LDS");
   const size_t ndeps_max = q->cap_deps;
   hipLaunchKernelGGL(queue_reset_kernel, dim3((unsigned)std::max<size_t>(1, std::min<size_t>(64, (ndeps_max + 255) / 256))),
-                     dim3(256), 0, st, q->d_counter, q->d_counter + (kXcd + 1) * kCtr, q->d_deps, q->d_hdr);
+                     dim3(256), 0, st, q->d_counter, q->d_counter + kStatus * kCtr, q->d_deps, q->d_hdr);
   QArgs a{};
   a.tasks = q->d_tasks;
   a.ptrs = q->d_ptrs;
   a.counter = q->d_counter;
   a.hdr = q->d_hdr;
   a.deps = q->d_deps;
-  a.status = q->d_counter + (kXcd + 1) * kCtr;
+  a.status = q->d_counter + kStatus * kCtr;
   a.spin_limit = q->spin_limit;
   a.tab = q->d_tab;
-  // the full grid even for few tasks: every XCD needs work-groups for its list
-  const int grid = q->grid;
-  if (q->groups_per_cu == 4)
-    hipLaunchKernelGGL(queue_kernel<4>, dim3(grid), dim3(kQThreads), kQLds, st, a);
-  else
-    hipLaunchKernelGGL(queue_kernel<2>, dim3(grid), dim3(kQThreads), kQLds, st, a);
-  hipError_t e = hipGetLastError();
+  // A captured launch runs the lists of whichever prepare is the latest at a
+  // replay, so it takes every kernel this queue's sizes can need; an eager one
+  // leaves out the kernels without a task.
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  const bool eager = hipStreamIsCapturing(st, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
+  auto has = [&](int l0, int l1, int lg) {
+    if (eager) return q->hdr.list_off[l0] < q->hdr.list_off[l1];
+    return q->max_lg >= lg && (lg == 0 || q->max_jobs << q->max_lg >= kLongPoints);
+  };
+  hipError_t e = hipSuccess;
+  if (has(QL_ROW15, QL_ROW14, 15)) e = queue_rows(a, QL_ROW15, q->ncu, st);
+  if (e == hipSuccess && has(QL_ROW14, QL_PAIR, 13)) e = queue_rows(a, QL_ROW14, q->ncu, st);
+  if (e == hipSuccess && has(QL_PAIR, kQLists, 16)) e = queue_pairs(a, eager ? q->hdr.list_off[kQLists] - q->hdr.list_off[QL_PAIR] : 0, q->ncu, st);
+  if (e == hipSuccess && has(0, QL_ROW15, 0)) {
+    // the full grid even for few tasks: every XCD needs work-groups for its list
+    const int grid = q->grid;
+    if (q->groups_per_cu == 4)
+      hipLaunchKernelGGL(queue_kernel<4>, dim3(grid), dim3(kQThreads), kQLds, st, a);
+    else
+      hipLaunchKernelGGL(queue_kernel<2>, dim3(grid), dim3(kQThreads), kQLds, st, a);
+    e = hipGetLastError();
+  }
   if (e != hipSuccess) {
     queue_set_err(hipGetErrorString(e));
     return -1;
   }
   // an eager launch is remembered so that the next prepare waits for it; a
   // captured one is not (the caller finishes its replays before a prepare)
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone) {
+  if (eager) {
     if (hipEventRecord(q->done, st) != hipSuccess) {
       queue_set_err("queue: event record failed");
       return -1;
@@ -724,7 +747,7 @@ int afft_gpu_queue_status(const afft_gpu_queue* qh) {
     return -1;
   }
   int v = 0;
-  if (hipDeviceSynchronize() != hipSuccess || hipMemcpy(&v, q->d_counter + (kXcd + 1) * kCtr, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess) {
+  if (hipDeviceSynchronize() != hipSuccess || hipMemcpy(&v, q->d_counter + kStatus * kCtr, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess) {
     queue_set_err("queue: status read failed");
     return -1;
   }

@@ -205,7 +205,7 @@ int afft_gpu_plan_describe(const afft_gpu_plan* plan, int i, char* buf, size_t l
 /* The last error message of the calling thread ("" if none). */
 const char* afft_gpu_last_error(void);
 
-/* ---- uneven batches in one persistent launch ------------------------------ */
+/* ---- uneven batches in persistent launches -------------------------------- */
 /* One job of a mixed batch: a 1-D FP32 transform of n = 2^log2n points,
  * interleaved complex, with afft's semantics for the kind:
  *   afft_gpu_c / afft_gpu_ci : n complex in, n complex out;
@@ -229,11 +229,13 @@ afft_gpu_queue* afft_gpu_queue_create(size_t max_jobs, int max_log2n, void* mem)
  * work).  It first waits for the previous eager launch of this queue; the
  * task, pointer and counter arrays were sized for max_jobs at create, and only
  * the scratch of the long jobs grows here.  Jobs of complex length <= 4096 run
- * in groups of one tile; longer ones as chains of tiles (real pre-pass,
- * four-step pass A, pass B, real post-pass) spread over the whole GPU.
+ * in groups of one tile; longer ones as whole rows (complex length up to 2^15)
+ * and four-step pass pairs (2^16) where their lengths add up to enough to fill
+ * the GPU, else as chains of tiles (real pre-pass, four-step pass A, pass B,
+ * real post-pass) spread over the whole GPU.
  * Returns the number of tasks, or -1. */
 int afft_gpu_queue_prepare(afft_gpu_queue* q, const afft_gpu_job* jobs, size_t njobs);
-/* Runs the prepared task list in one persistent launch on `stream`.  Issues
+/* Runs the prepared task lists in persistent launches on `stream`.  Issues
  * kernels only, so it can be captured in a HIP graph and replayed.  A launch
  * and every replay of a captured one run the task list of the LATEST prepare
  * (the list offsets and counts are read from device memory at run time): a
