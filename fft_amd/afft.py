@@ -11,6 +11,7 @@ stream-aware extension (include/afft_gpu.h)."""
 from __future__ import annotations
 
 import ctypes
+import math
 import sys
 
 import numpy as np
@@ -23,7 +24,7 @@ def _half_count(dims) -> int:
     """Complex elements of a real transform's complex side: dim 0 (after unit
     dims are dropped) becomes N0/2+1 (fft_internal.hpp:215-219)."""
     s = [int(d) for d in dims if int(d) != 1] or [1]
-    return (s[0] // 2 + 1) * int(np.prod(s[1:], dtype=np.int64))
+    return (s[0] // 2 + 1) * math.prod(s[1:])
 
 
 def required_counts(kind: str, dims, fmt: int, batch: int = 1):
@@ -31,7 +32,7 @@ def required_counts(kind: str, dims, fmt: int, batch: int = 1):
     transforms back to back (0: the argument is not read or written).  Real
     kinds take (src, dst_re, dst_im) and (src_re, src_im, dst); the tuple is
     in that argument order."""
-    n = int(np.prod([int(d) for d in dims], dtype=np.int64))
+    n = math.prod(int(d) for d in dims)
     m = _half_count(dims)
     il = int(fmt) == afft_interleaved
     b = int(batch)
