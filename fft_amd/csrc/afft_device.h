@@ -253,6 +253,7 @@ AFGPU_SCHED(32768, 0, 32, 3, 32, 32, 32)
 AFGPU_SCHED(512, 1, 32, 2, 32, 16)
 AFGPU_SCHED(1024, 1, 32, 2, 32, 32)
 AFGPU_SCHED(2048, 1, 32, 3, 32, 32, 2)
+AFGPU_SCHED(8192, 1, 32, 3, 32, 32, 8)
 AFGPU_SCHED(16384, 1, 32, 3, 32, 32, 16)
 #undef AFGPU_SCHED
 

@@ -738,6 +738,9 @@ constexpr size_t tile_lds_bytes() {
 template <typename T, int L, int CT, bool COLMAP, bool STORE_T, int SV, bool HX>
 constexpr int pass_min_waves() {
   constexpr int nt = PassShape<L, CT, SV>::NT;
+  constexpr size_t lds = tile_lds_bytes<T, L, CT, COLMAP, STORE_T, SV, HX>();
+  // 256-thread rows of 32 elements a thread (8192 points): four groups per CU
+  if (HX && nt == 256 && 4 * lds <= 160 * 1024) return 4;
   constexpr int groups = (HX && 2 * tile_lds_bytes<T, L, CT, COLMAP, STORE_T, SV, HX>() <= 160 * 1024) ? 2 : 1;
   return groups * nt / 256 > 1 ? groups * nt / 256 : 1;
 }

@@ -408,7 +408,17 @@ struct Builder {
   // pref_ct > 0: a tile tried before the defaults (split-addressed column
   // passes ask for wide tiles, whose 4-byte re / im accesses then still cover
   // whole 256-byte row segments)
-  bool fft_pass(PassRec* r, int L, int colmap, int epi, int store_t, int pref_ct = 0) {
+  //
+  // rows: rows of a plain row pass in one user transform.  Rows of 16384 points
+  // and the r2c of 16384 reals run radix-32 stages in half the LDS (512 and 256
+  // threads, two and four groups per CU, so one's loads run beside another's
+  // butterflies) once there are more rows than the full-LDS groups of one round
+  // on the chip hold.  us, radix-16 / radix-32: c2c 16384 256 rows 18.3 / 23.8,
+  // 300 30.5 / 28.5, 2048 135.7 / 132.5; r2c 32768 256 23.2 / 25.1, 300 36.6 /
+  // 28.8, 2048 172 / 142; c2r 32768 256 22.6 / 25.7, 300 35.7 / 33.1, 2048 176
+  // / 167; r2c 16384 512 21.0 / 21.9, 1024 37.2 / 30.8, 4096 139 / 122.  8192
+  // points c2c and c2r lose (114 / 117, 139 / 150) and have no such kernel.
+  bool fft_pass(PassRec* r, int L, int colmap, int epi, int store_t, int pref_ct = 0, idx_t rows = 1) {
     // tile: the variant's choice for column / transposed-store passes, else
     // the compiled default; schedule: radix-32 where compiled unless the
     // variant opts out; then the half-LDS kernel of that shape if one exists
@@ -425,6 +435,8 @@ struct Builder {
     // 64 x 2^20 direction for two 16-column groups; they stay a variant,
     // col_tile = 32)
     const bool wide = want <= 0 && colmap && P.var.half_lds >= 0 && L != 1024;
+    const bool few_rows = !colmap && !store_t && L >= 8192 && P.var.sched <= 0 &&
+                          rows * P.batch <= (L == 8192 ? 512 : 256);
     // (the dim-0 real column passes too: r2c 256^3 0.135 -> 0.080 ms, 128^3 x 8
     // 0.124 -> 0.076, 256 x 512 x 256 0.320 -> 0.160; c2r 256^3 0.0885 -> 0.085,
     // but c2r with 64-point columns 0.087 -> 0.092, so those keep the default
@@ -440,7 +452,7 @@ struct Builder {
     for (const Cand& c : cands)
       for (int sv : {1, 0})
         for (int hx : {1, 0}) {
-          if (v || c.ct <= 0 || (c.hx_only && !hx) || (sv && P.var.sched < 0) || (hx && P.var.half_lds < 0))
+          if (v || c.ct <= 0 || (c.hx_only && !hx) || (sv && (P.var.sched < 0 || few_rows)) || (hx && P.var.half_lds < 0))
             continue;
           v = find_pass<T>(L, c.ct, colmap, epi, store_t, sv, hx);
         }
@@ -509,7 +521,7 @@ struct Builder {
 
     if (inner == 1 && n <= row_max()) {
       PassRec* r = add();
-      if (!r || !fft_pass(r, (int)n, 0, EPI_PLAIN, 0)) return;
+      if (!r || !fft_pass(r, (int)n, 0, EPI_PLAIN, 0, 0, outer_u)) return;
       r->in = in;
       r->out = out;
       r->in.s_j = 1;
@@ -2551,6 +2563,7 @@ int stage_list(int L, int sv, int* radix, int* ns) {
       case 512: return fill_stages<512, 1>(radix, ns);
       case 1024: return fill_stages<1024, 1>(radix, ns);
       case 2048: return fill_stages<2048, 1>(radix, ns);
+      case 8192: return fill_stages<8192, 1>(radix, ns);
       case 16384: return fill_stages<16384, 1>(radix, ns);
       default: return 0;
     }
