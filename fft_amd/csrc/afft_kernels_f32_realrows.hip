@@ -1,0 +1,3 @@
+// FP32 row passes with a real pass.
+#define AFGPU_PART 3
+#include "afft_kernels_f32.hip"

@@ -80,7 +80,8 @@ struct PassParams {
   int tw4_log2n;          // > 0 (FP32): compute W_N^m, N = 2^tw4_log2n, instead of the table lookup
   const cx<T>* real_tw;   // W_{2L}^k, k < L (EPI_C2R4: W_{2h}^k, k < h)
   idx_t real_h;           // EPI_C2R4: h, the number of complex points
-  // Byte extents of the in / out regions of one batch entry (fast path only).
+  // Byte extents of the in / out regions of one batch entry, of each of its two
+  // arrays where it is split (buffer access only).
   unsigned in_bytes, out_bytes;
   // Optional per-column buffers (uneven batches): column c reads from
   // col_ptrs[2c] and writes to col_ptrs[2c+1], both interleaved, with the
@@ -307,12 +308,14 @@ struct PassShape {
 // One tile (CT columns) of a pass, executed by the NT = CT * L/E threads
 // tid = 0..NT-1 of a work-group, with `lds` holding CT * LdsLen<L> entries.
 // ---- element access ---------------------------------------------------------
-// Generic access follows PassParams in full (split / interleaved, one-array
-// split, per-column buffers).  FAST access is for interleaved data on both
-// sides: one buffer resource per tile side (base and byte extent uniform over
-// the work-group, so reads past the extent return 0 and writes past it are
-// dropped) and 32-bit byte offsets per element, which saves the 64-bit address
-// arithmetic of every load and store.
+// MODE 0, generic access, follows PassParams in full (split / interleaved,
+// one-array split, per-column buffers, any extent).  MODE 1 is for interleaved
+// data on both sides: one buffer resource per tile side (base and byte extent
+// uniform over the work-group, so reads past the extent return 0 and writes
+// past it are dropped) and 32-bit byte offsets per element, which saves the
+// 64-bit address arithmetic of every load and store.  MODE 2 is the same where
+// a side is split: one resource per array, and the format and cache policy
+// chosen once per phase instead of by branches around every access.
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
@@ -350,6 +353,27 @@ __device__ __forceinline__ void buf_st(cx<double> v, __amdgpu_buffer_rsrc_t r, u
   __builtin_amdgcn_raw_buffer_store_b128(w, r, off, 0, AUX);
 }
 
+// one part (real or imaginary) of an element
+template <typename T, int AUX>
+__device__ __forceinline__ T buf_ld1(__amdgpu_buffer_rsrc_t r, unsigned off) {
+  if constexpr (std::is_same_v<T, float>) {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, AUX));
+  } else {
+    u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, AUX);
+    return __hiloint2double(w.y, w.x);
+  }
+}
+template <int AUX>
+__device__ __forceinline__ void buf_st1(float v, __amdgpu_buffer_rsrc_t r, unsigned off) {
+  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, off, 0, AUX);
+}
+template <int AUX>
+__device__ __forceinline__ void buf_st1(double v, __amdgpu_buffer_rsrc_t r, unsigned off) {
+  unsigned long long a = __double_as_longlong(v);
+  u32x2 w = {(unsigned)a, (unsigned)(a >> 32)};
+  __builtin_amdgcn_raw_buffer_store_b64(w, r, off, 0, AUX);
+}
+
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
 }
@@ -364,7 +388,12 @@ __device__ __forceinline__ cx<T> real_twiddle(const cx<T>* __restrict__ tab, int
     return tab[k];
 }
 
-// A cache policy known only at run time (one branch per access).
+// How a side of a tile is accessed, as a compile-time number: bit 1 set =
+// non-temporal, bit 2 set = separate real and imaginary arrays.
+enum { POL_NT = 2, POL_SPLIT = 4 };
+
+// The same with the cache policy known only at run time (one branch per access).
+template <int SPLIT>
 struct RtPol {
   int nt;
 };
@@ -372,7 +401,7 @@ struct RtPol {
 // One tile (CT columns) of a pass, executed by the NT = CT * L/E threads
 // tid = 0..NT-1 of a work-group, with `lds` holding CT * LdsLen<L> entries.
 
-template <typename T, int L, int CT, bool COLMAP, int EPI, bool STORE_T, bool FAST = false, int SV = 0, bool HX = false>
+template <typename T, int L, int CT, bool COLMAP, int EPI, bool STORE_T, int MODE = 0, int SV = 0, bool HX = false>
 __device__ __forceinline__ void fft_tile(const PassParams<T>& p, int tile, int tid, cx<T>* __restrict__ lds) {
   static_assert(EPI != EPI_C2R4 || (COLMAP && !STORE_T), "the paired load is for four-step column passes");
   using PS = PassShape<L, CT, SV, (!COLMAP && STORE_T) ? (HX ? (int)sizeof(T) : 2 * (int)sizeof(T)) : 0>;
@@ -380,6 +409,7 @@ __device__ __forceinline__ void fft_tile(const PassParams<T>& p, int tile, int t
   constexpr int TPT = PS::TPT;
   constexpr int LL = PS::LL;
   constexpr unsigned ES = sizeof(cx<T>);
+  constexpr bool FAST = MODE != 0;
 
   const int c = COLMAP ? (tid % CT) : (tid / TPT);
   const int t = COLMAP ? (tid / CT) : (tid % TPT);
@@ -410,18 +440,26 @@ __device__ __forceinline__ void fft_tile(const PassParams<T>& p, int tile, int t
   T* out_re = p.out_re;
   T* out_im = p.out_im;
   idx_t ib = 0, ob = 0;
-  // fast addressing: per-side resource + 32-bit byte offsets
+  // fast addressing: per-side resources + 32-bit byte offsets (bytes per
+  // element: ES interleaved, half of that in each of two split arrays)
   __amdgpu_buffer_rsrc_t rin = make_rsrc(p.in_re, 0u), rout = make_rsrc(p.out_re, 0u);
+  __amdgpu_buffer_rsrc_t rin_im = rin, rout_im = rout;
   unsigned in0 = 0, out0 = 0, js8 = 0, ks8 = 0;
+  const unsigned esi = MODE == 2 && !p.in_il ? ES / 2 : ES;
+  const unsigned eso = MODE == 2 && !p.out_il ? ES / 2 : ES;
   if constexpr (FAST) {
-    rin = make_rsrc(reinterpret_cast<const cx<T>*>(p.in_re) + ((idx_t)bhi * p.in_bs + (idx_t)blo * p.in_bs2),
-                    p.in_bytes);
-    rout = make_rsrc(reinterpret_cast<const cx<T>*>(p.out_re) + ((idx_t)bhi * p.out_bs + (idx_t)blo * p.out_bs2),
-                     p.out_bytes);
-    in0 = (unsigned)col * (unsigned)p.in_cs * ES;
-    out0 = (unsigned)col * (unsigned)p.out_cs * ES;
-    js8 = (unsigned)p.in_js * ES;
-    ks8 = (unsigned)p.out_ks * ES;
+    const idx_t bi = ((idx_t)bhi * p.in_bs + (idx_t)blo * p.in_bs2) * esi;
+    const idx_t bo = ((idx_t)bhi * p.out_bs + (idx_t)blo * p.out_bs2) * eso;
+    rin = make_rsrc(reinterpret_cast<const char*>(p.in_re) + bi, p.in_bytes);
+    rout = make_rsrc(reinterpret_cast<const char*>(p.out_re) + bo, p.out_bytes);
+    if constexpr (MODE == 2) {
+      rin_im = make_rsrc(reinterpret_cast<const char*>(p.in_im) + bi, p.in_bytes);
+      rout_im = make_rsrc(reinterpret_cast<const char*>(p.out_im) + bo, p.out_bytes);
+    }
+    in0 = (unsigned)col * (unsigned)p.in_cs * esi;
+    out0 = (unsigned)col * (unsigned)p.out_cs * eso;
+    js8 = (unsigned)p.in_js * esi;
+    ks8 = (unsigned)p.out_ks * eso;
   } else {
     ib = (idx_t)bhi * p.in_bs + (idx_t)blo * p.in_bs2 + (idx_t)col * p.in_cs;
     ob = (idx_t)bhi * p.out_bs + (idx_t)blo * p.out_bs2 + (idx_t)col * p.out_cs;
@@ -436,13 +474,28 @@ __device__ __forceinline__ void fft_tile(const PassParams<T>& p, int tile, int t
       }
     }
   }
-  // element j of this column / bin k of this column.  POL is the cache policy
-  // of the fast path's buffer accesses (2 = non-temporal), chosen once per
-  // phase below so that no access carries a branch of its own.
+  // element j of this column / bin k of this column.  polc is the format and
+  // cache policy of the fast path's buffer accesses, chosen once per phase below
+  // so that no access carries a branch of its own.
+  auto ld_buf = [&](auto polc, unsigned off) AFGPU_INLINE -> cx<T> {
+    constexpr int pol = decltype(polc)::value;
+    if constexpr (pol & POL_SPLIT)
+      return {buf_ld1<T, pol & POL_NT>(rin, off), buf_ld1<T, pol & POL_NT>(rin_im, off)};
+    else
+      return buf_ld<T, pol & POL_NT>(rin, off);
+  };
+  auto st_buf = [&](auto polc, unsigned off, cx<T> z) AFGPU_INLINE {
+    constexpr int pol = decltype(polc)::value;
+    if constexpr (pol & POL_SPLIT) {
+      buf_st1<pol & POL_NT>(z.x, rout, off);
+      buf_st1<pol & POL_NT>(z.y, rout_im, off);
+    } else {
+      buf_st<pol & POL_NT>(z, rout, off);
+    }
+  };
   auto load = [&](auto polc, int j) AFGPU_INLINE -> cx<T> {
     if constexpr (FAST) {
-      const unsigned off = in0 + (unsigned)j * js8;
-      return buf_ld<T, decltype(polc)::value>(rin, off);
+      return ld_buf(polc, in0 + (unsigned)j * js8);
     } else {
       return ld_elem(in_re, in_im, p.in_il, ib + (idx_t)j * p.in_js, p.in_nt);
     }
@@ -450,7 +503,7 @@ __device__ __forceinline__ void fft_tile(const PassParams<T>& p, int tile, int t
   // element at offset e (elements) from the batch entry's base (EPI_C2R4)
   auto load_at = [&](auto polc, idx_t e) AFGPU_INLINE -> cx<T> {
     if constexpr (FAST) {
-      return buf_ld<T, decltype(polc)::value>(rin, (unsigned)e * ES);
+      return ld_buf(polc, (unsigned)e * esi);
     } else {
       return ld_elem(p.in_re, p.in_im, p.in_il, (idx_t)bhi * p.in_bs + (idx_t)blo * p.in_bs2 + e, p.in_nt);
     }
@@ -459,27 +512,32 @@ __device__ __forceinline__ void fft_tile(const PassParams<T>& p, int tile, int t
     if (p.swap_out) z = swapri(z);
     if constexpr (FAST) {
       const unsigned off = out0 + (unsigned)k * ks8;
-      if constexpr (std::is_same_v<decltype(polc), RtPol>) {
+      if constexpr (std::is_same_v<decltype(polc), RtPol<0>> || std::is_same_v<decltype(polc), RtPol<POL_SPLIT>>) {
+        constexpr int split = std::is_same_v<decltype(polc), RtPol<POL_SPLIT>> ? POL_SPLIT : 0;
         if (polc.nt)
-          buf_st<2>(z, rout, off);
+          st_buf(std::integral_constant<int, POL_NT | split>{}, off, z);
         else
-          buf_st<0>(z, rout, off);
+          st_buf(std::integral_constant<int, split>{}, off, z);
       } else {
-        buf_st<decltype(polc)::value>(z, rout, off);
+        st_buf(polc, off, z);
       }
     } else {
       st_elem(out_re, out_im, p.out_il, ob + (idx_t)k * p.out_ks, z, p.out_nt);
     }
   };
 
-  // runs f(pol) with pol = the compile-time cache policy for a side whose
-  // streaming flag is nt
-  auto with_pol = [&](bool nt, auto&& f) AFGPU_INLINE {
-    if constexpr (FAST) {
-      if (nt)
-        f(std::integral_constant<int, 2>{});
-      else
-        f(std::integral_constant<int, 0>{});
+  // runs f(pol) with pol = the compile-time policy of a side that is split or
+  // not and whose streaming flag is nt
+  auto with_pol = [&](int il, bool nt, auto&& f) AFGPU_INLINE {
+    if (MODE == 2 && !il) {
+      if constexpr (MODE == 2) {
+        if (nt)
+          f(std::integral_constant<int, POL_SPLIT | POL_NT>{});
+        else
+          f(std::integral_constant<int, POL_SPLIT>{});
+      }
+    } else if (FAST && nt) {
+      f(std::integral_constant<int, POL_NT>{});
     } else {
       f(std::integral_constant<int, 0>{});
     }
@@ -487,7 +545,7 @@ __device__ __forceinline__ void fft_tile(const PassParams<T>& p, int tile, int t
 
   cx<T> v[E];
   if (active) {
-    with_pol(p.in_nt, [&](auto pol) AFGPU_INLINE {
+    with_pol(p.in_il, p.in_nt, [&](auto pol) AFGPU_INLINE {
       if constexpr (EPI == EPI_C2R4) {
         // Z[k] = (X[k] + conj X[h-k]) - i conj(W_2h^k) (conj X[h-k] - X[k]),
         // Z[0] = (Re X[0] + Re X[h]) + i (Re X[0] - Re X[h]); eight elements at
@@ -557,10 +615,16 @@ __device__ __forceinline__ void fft_tile(const PassParams<T>& p, int tile, int t
   // (fewer live registers in their twiddled store); row tiles keep one branch
   // per store, which measured fewer spills in the transposed store.
   auto with_out_pol = [&](auto&& f) AFGPU_INLINE {
-    if constexpr (COLMAP)
-      with_pol(p.out_nt, f);
-    else
-      f(RtPol{p.out_nt});
+    if constexpr (COLMAP || (MODE == 2 && !STORE_T)) {
+      with_pol(p.out_il, p.out_nt, f);
+    } else if constexpr (MODE == 2) {
+      if (p.out_il)
+        f(RtPol<0>{p.out_nt});
+      else
+        f(RtPol<POL_SPLIT>{p.out_nt});
+    } else {
+      f(RtPol<0>{p.out_nt});
+    }
   };
   with_out_pol([&](auto pol) AFGPU_INLINE {
     if constexpr (EPI == EPI_R2C) {
@@ -677,7 +741,7 @@ __device__ __forceinline__ void fft_tile(const PassParams<T>& p, int tile, int t
         const int colb = col0 + c2;
         // re-aim the output at column colb (the thread's column changes here)
         if constexpr (FAST) {
-          out0 = (unsigned)colb * (unsigned)p.out_cs * ES;
+          out0 = (unsigned)colb * (unsigned)p.out_cs * eso;
         } else {
           ob = (idx_t)bhi * p.out_bs + (idx_t)blo * p.out_bs2 + (idx_t)colb * p.out_cs;
           out_re = p.out_re;
@@ -745,7 +809,7 @@ constexpr int pass_min_waves() {
   return groups * nt / 256 > 1 ? groups * nt / 256 : 1;
 }
 
-template <typename T, int L, int CT, bool COLMAP, int EPI, bool STORE_T, bool FAST, int SV, bool HX>
+template <typename T, int L, int CT, bool COLMAP, int EPI, bool STORE_T, int MODE, int SV, bool HX>
 __global__ void __launch_bounds__((PassShape<L, CT, SV>::NT), (pass_min_waves<T, L, CT, COLMAP, STORE_T, SV, HX>()))
     fft_pass_kernel(PassParams<T> p) {
   extern __shared__ __align__(16) unsigned char afgpu_smem[];
@@ -764,7 +828,7 @@ __global__ void __launch_bounds__((PassShape<L, CT, SV>::NT), (pass_min_waves<T,
       tile = b * p.col_tiles + ((B & 8) ? p.col_tiles - 1 - pp : pp);
     }
   }
-  fft_tile<T, L, CT, COLMAP, EPI, STORE_T, FAST, SV, HX>(p, tile, threadIdx.x,
+  fft_tile<T, L, CT, COLMAP, EPI, STORE_T, MODE, SV, HX>(p, tile, threadIdx.x,
                                                          reinterpret_cast<cx<T>*>(afgpu_smem));
 }
 

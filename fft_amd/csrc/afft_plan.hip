@@ -1655,9 +1655,9 @@ int tw4_log2n(const PassRec& r) {
   return (sizeof(T) == 4 && n >= 8 && n <= ((idx_t)1 << 27) && (n & (n - 1)) == 0) ? ilog2(n) : 0;
 }
 
-// `fast` tells whether the buffer-resource path applies.
+// `mode` is the addressing the tile can use (fft_tile's MODE).
 template <typename T>
-bool fft_params(const PassRec& r, const Bufs<T>& B, idx_t start, idx_t cnt, PassParams<T>& p, bool& fast) {
+bool fft_params(const PassRec& r, const Bufs<T>& B, idx_t start, idx_t cnt, PassParams<T>& p, int& mode) {
   const T *ire, *iim, *ore_c, *oim_c;
   resolve(r.in, B, start, ire, iim);
   resolve(r.out, B, start, ore_c, oim_c);
@@ -1712,18 +1712,18 @@ bool fft_params(const PassRec& r, const Bufs<T>& B, idx_t start, idx_t cnt, Pass
   // path needs it below 4 GiB
   const idx_t lin = (idx_t)r.L + (r.epi == EPI_C2R ? 1 : 0);
   const idx_t lout = (idx_t)r.L + (r.epi == EPI_R2C ? 1 : 0);
-  idx_t ext_in = ((ncol - 1) * r.in.s_c + (lin - 1) * r.in.s_j + 1) * (idx_t)sizeof(cx<T>);
+  const idx_t esi = r.in.il ? sizeof(cx<T>) : sizeof(T), eso = r.out.il ? sizeof(cx<T>) : sizeof(T);
+  idx_t ext_in = ((ncol - 1) * r.in.s_c + (lin - 1) * r.in.s_j + 1) * esi;
   if (r.epi == EPI_C2R4) {
     // the paired load reaches bin h of each batch entry
     p.real_h = r.rr_h;
-    ext_in = std::max(ext_in, (r.rr_h + 1) * (idx_t)sizeof(cx<T>));
+    ext_in = std::max(ext_in, (r.rr_h + 1) * esi);
   }
-  const idx_t ext_out = ((ncol - 1) * r.out.s_c + (lout - 1) * r.out.s_j + 1) * (idx_t)sizeof(cx<T>);
-  const bool fast_ok = r.in.il && r.out.il && ext_in > 0 && ext_out > 0 && ext_in < ((idx_t)1 << 32) &&
-                       ext_out < ((idx_t)1 << 32);
-  p.in_bytes = fast_ok ? (unsigned)ext_in : 0u;
-  p.out_bytes = fast_ok ? (unsigned)ext_out : 0u;
-  fast = fast_ok;
+  const idx_t ext_out = ((ncol - 1) * r.out.s_c + (lout - 1) * r.out.s_j + 1) * eso;
+  const bool buffers = ext_in > 0 && ext_out > 0 && ext_in < ((idx_t)1 << 32) && ext_out < ((idx_t)1 << 32);
+  p.in_bytes = buffers ? (unsigned)ext_in : 0u;
+  p.out_bytes = buffers ? (unsigned)ext_out : 0u;
+  mode = !buffers ? 0 : r.in.il && r.out.il ? 1 : 2;
   return true;
 }
 
@@ -1777,9 +1777,9 @@ bool run_pass(const PassRec& r, const Bufs<T>& B, idx_t start, idx_t cnt, hipStr
   if (r.type == PT_FFT) {
     const PassVariant<T>* v = (const PassVariant<T>*)r.variant;
     PassParams<T> p;
-    bool fast = false;
-    if (!fft_params<T>(r, B, start, cnt, p, fast)) return false;
-    HIP_OK(v->launch(p, st, fast));
+    int mode = 0;
+    if (!fft_params<T>(r, B, start, cnt, p, mode)) return false;
+    HIP_OK(v->launch(p, st, mode));
     return true;
   }
   if (r.type == PT_REALROWS) {

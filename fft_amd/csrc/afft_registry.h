@@ -9,7 +9,7 @@
 namespace afgpu {
 
 template <typename T>
-using PassLaunchFn = hipError_t (*)(const PassParams<T>&, hipStream_t, bool fast);
+using PassLaunchFn = hipError_t (*)(const PassParams<T>&, hipStream_t, int mode);
 
 template <typename T>
 struct PassVariant {
@@ -35,11 +35,15 @@ PassList<float> pass_part<float, 1>();
 template <>
 PassList<float> pass_part<float, 2>();
 template <>
+PassList<float> pass_part<float, 3>();
+template <>
 PassList<double> pass_part<double, 0>();
 template <>
 PassList<double> pass_part<double, 1>();
 template <>
 PassList<double> pass_part<double, 2>();
+template <>
+PassList<double> pass_part<double, 3>();
 
 // Looks up the compiled variant; returns nullptr when none exists.
 template <typename T>
