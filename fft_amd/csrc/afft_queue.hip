@@ -647,8 +647,7 @@ int afft_gpu_queue_prepare(afft_gpu_queue* qh, const afft_gpu_job* jobs, size_t 
         t.kind = j.kind;
         t.lg = lg;
         t.count = 1;
-        t.src = j.src;
-        t.dst = j.dst;
+        t.set_buffers(j.src, j.dst);
         q->h_tasks.push_back(t);
       }
   };

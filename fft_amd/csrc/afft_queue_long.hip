@@ -31,7 +31,8 @@ struct QRec {
 };
 __device__ __forceinline__ QRec q_rec(const QArgs& a, int i) {
   const QConst<QTask> t = q_const(a.tasks) + i;
-  return {t->kind, t->lg, t->src, t->dst};
+  auto pair = [](int lo, int hi) AFGPU_INLINE { return (unsigned long long)(unsigned)hi << 32 | (unsigned)lo; };
+  return {t->kind, t->lg, pair(t->first, t->job), pair(t->tile, t->need)};
 }
 
 // One row of 2^lg points, addressed through buffer resources.
