@@ -68,11 +68,14 @@ constexpr int kRealTile = 2048;  // bin pairs per real-pass tile
 constexpr int kLag = 128;        // default jobs between consecutive steps of one chain (per XCD list)
 // Long jobs (2^13 complex points and more) run as whole rows and pass pairs
 // (afft_queue_long.hip) from this many complex points of them in all, as chains
-// below.  Chains against rows and pairs, in us: 100 jobs of 2^13..2^15 (1.9 M
-// points) 46 / 85, 300 (5.6 M) 69 / 91, 700 of 2^6..2^16 (6.5 M) 94 / 115,
-// 1000 (9.3 M) 120 / 124, 500 of 2^13..2^15 (9.4 M) 110 / 98, 1000 (19 M)
-// 190 / 124, 300 of 2^16 (17 M) 179 / 129, 3000 of 2^6..2^16 (28 M) 295 / 246.
-constexpr size_t kLongPoints = (size_t)10 << 20;
+// below: from kLongPoints where there are only rows or only pairs, from
+// kLongPointsMixed where both occur (three launches, each with its last round).
+// Chains against rows and pairs, in us: 300 jobs of 2^13..2^15 (5 M points)
+// 69 / 91, 500 (8 M) 83 / 95, 700 (10.7 M) 125 / 101, 1000 (15 M) 177 / 121;
+// 190 jobs of 2^16 (10.2 M) 114 / 102, 300 (16 M) 176 / 127; 1000 of 2^6..2^16
+// (9 M, both) 104 / 120, 1200 (10.6 M) 126 / 131, 1350 (11.9 M) 137 / 134, 1500
+// (12.9 M) 150 / 138, 3000 283 / 240, 10,000 907 / 604.
+constexpr size_t kLongPoints = (size_t)10 << 20, kLongPointsMixed = (size_t)12 << 20;
 constexpr int kStatus = kQLists;  // counter slot of the status flag
 
 template <int L>
@@ -530,7 +533,7 @@ int afft_gpu_queue_prepare(afft_gpu_queue* qh, const afft_gpu_job* jobs, size_t 
   size_t points = 0;
   for (size_t i : rows) points += (size_t)1 << (jobs[i].log2n - (jobs[i].kind >= afft_gpu_r ? 1 : 0));
   points += pairs.size() << 16;
-  if (points < kLongPoints) {
+  if (points < (rows.empty() || pairs.empty() ? kLongPoints : kLongPointsMixed)) {
     big.swap(rows);
     big.insert(big.end(), pairs.begin(), pairs.end());
     pairs.clear();

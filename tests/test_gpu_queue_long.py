@@ -41,7 +41,8 @@ def lengths(spec):
     return sum(1 << (lg - (1 if k in (R, RI) else 0)) for k, lg in spec)
 
 
-LIMIT = 10 << 20  # complex points of long jobs from which they leave the chains
+LIMIT = 10 << 20  # complex points of long jobs of one class from which they leave the chains
+MIXED = 12 << 20  # of rows and pairs
 CASES = {
     # one job short of the rule, and on it
     "rows15 below": [(C, 15)] * (LIMIT // 32768 - 1),
@@ -50,7 +51,9 @@ CASES = {
     "rows14 13": [(C, 14), (CI, 14), (C, 13)] * 270,
     "pairs one group": [(C, 16), (CI, 16)] * 81,
     "pairs three groups": [(C, 16)] * 450 + [(CI, 16)] * 449,
-    "all": [(k, lg) for k in (C, CI, R, RI) for lg in (13, 14, 15, 16)] * 24 + [(C, 5), (R, 9), (RI, 13), (CI, 12)],
+    "rows and pairs below": [(C, 15)] * (MIXED // 32768 - 3) + [(CI, 16)],
+    "rows and pairs at": [(C, 15)] * (MIXED // 32768 - 2) + [(CI, 16)],
+    "all": [(k, lg) for k in (C, CI, R, RI) for lg in (13, 14, 15, 16)] * 40 + [(C, 5), (R, 9), (RI, 13), (CI, 12)],
 }
 
 
@@ -89,7 +92,7 @@ def test_captured_launch_runs_the_latest_prepare(G):
     import torch
     from fft_amd.afft import Queue
     few = [(C, 15), (R, 16), (CI, 16), (RI, 15), (C, 8)]
-    many = [(C, 15), (CI, 16), (R, 16), (RI, 15), (C, 14), (R, 14), (C, 7)] * 70
+    many = [(C, 15), (CI, 16), (R, 16), (RI, 15), (C, 14), (R, 14), (C, 7)] * 80
     none = [(C, 10), (R, 11)] * 9
     s = torch.cuda.Stream()
     q = Queue(len(many), 16)
