@@ -395,12 +395,29 @@ struct Builder {
   // half-LDS kernels off.
   idx_t row_max() const { return P.var.half_lds < 0 ? max_row_len_full<T>() : max_row_len<T>(); }
 
+  // Few points: an FP32 call whose passes, with the tiles that suit long
+  // batches, are fewer groups than the chip has CUs (a single 2^16-point
+  // transform ran 16 and 8 groups, a single 2^20 64 and 128).  Such a four-step
+  // takes balanced factors and the narrowest full-LDS radix-16 tiles instead:
+  // more, smaller groups, no second exchange.  us, before / after, FP32 c2c:
+  // 2^16 x 1 16.9 / 15.0, 2^17 x 1 19.5 / 14.8, x 4 21.3 / 16.2, 2^18 x 1 20.1 /
+  // 15.5, x 4 24.3 / 20.2, 2^19 x 1 26.1 / 19.0, x 2 30.4 / 22.1, 2^20 x 1 28.7 /
+  // 24.3, x 2 33.4 / 29.4, 2^21 x 1 37 / 32, 2^22 x 1 57.5 / 45.2; 2^20 x 16 and
+  // 2^22 x 2 are faster with the wide tiles.  A variant that names a schedule,
+  // an exchange or a split is followed as it is.
+  bool few_points(idx_t points, int lg_limit) const {
+    const Variant& v = P.var;
+    return sizeof(T) == 4 && P.mode == afft_gpu_mode_fma && v.sched == 0 && v.half_lds == 0 && v.row_log2 == 0 &&
+           v.fused <= 0 && points <= ((idx_t)1 << lg_limit);
+  }
+
   // Row length n2 of the 1-D four-step n = n1 * n2: 1024-point rows up to
   // 2^20, but columns of at least 64 points (a pass A over 16- or 32-point
   // columns measured 1.29 TB/s for FP64 2^14, 2.84 as 64 x 256; FP64 2^15
   // 2.39 -> 2.75 as 64 x 512); longer rows beyond 2^20.
-  idx_t row_len_1d(idx_t n) const {
+  idx_t row_len_1d(idx_t n, bool few = false) const {
     if (P.var.row_log2 > 0) return P.var.row_log2 < 40 ? (idx_t)1 << P.var.row_log2 : 0;
+    if (few && n <= ((idx_t)1 << 20)) return n <= 32768 ? 512 : (idx_t)1 << (ilog2(n) / 2);
     if (n <= ((idx_t)1 << 20)) return std::min<idx_t>(1024, std::max<idx_t>(2, n / 64));
     return std::max<idx_t>(2048, n / max_col_len<T>());
   }
@@ -418,7 +435,7 @@ struct Builder {
   // 28.8, 2048 172 / 142; c2r 32768 256 22.6 / 25.7, 300 35.7 / 33.1, 2048 176
   // / 167; r2c 16384 512 21.0 / 21.9, 1024 37.2 / 30.8, 4096 139 / 122.  8192
   // points c2c and c2r lose (114 / 117, 139 / 150) and have no such kernel.
-  bool fft_pass(PassRec* r, int L, int colmap, int epi, int store_t, int pref_ct = 0, idx_t rows = 1) {
+  bool fft_pass(PassRec* r, int L, int colmap, int epi, int store_t, int pref_ct = 0, idx_t rows = 1, bool few = false) {
     // tile: the variant's choice for column / transposed-store passes, else
     // the compiled default; schedule: radix-32 where compiled unless the
     // variant opts out; then the half-LDS kernel of that shape if one exists
@@ -435,6 +452,12 @@ struct Builder {
     // 64 x 2^20 direction for two 16-column groups; they stay a variant,
     // col_tile = 32)
     const bool wide = want <= 0 && colmap && P.var.half_lds >= 0 && L != 1024;
+    if (few) {
+      // 8 columns / rows of 512 points and more, 16 of shorter ones
+      const int ct = L >= 512 ? 8 : 16;
+      v = find_pass<T>(L, want > 0 ? want : ct, colmap, epi, store_t, 0, 0);
+      if (!v) v = find_pass<T>(L, deflt, colmap, epi, store_t, 0, 0);
+    }
     const bool few_rows = !colmap && !store_t && L >= 8192 && P.var.sched <= 0 &&
                           rows * P.batch <= (L == 8192 ? 512 : 256);
     // (the dim-0 real column passes too: r2c 256^3 0.135 -> 0.080 ms, 128^3 x 8
@@ -519,7 +542,11 @@ struct Builder {
     if (out.role < R_SCR && out.s_u == 0) out.s_u = tens;
     const int tmp_role = (in.role == R_SCR || out.role == R_SCR) ? R_SCR2 : R_SCR;
 
-    if (inner == 1 && n <= row_max()) {
+    const bool few = inner == 1 && few_points(n * outer_u * P.batch, n >= ((idx_t)1 << 20) ? 22 : 21);
+    // a single 32768-point transform: one group of one CU takes 25 us, the
+    // four-step over 64 groups 14
+    const bool lone = few && n == 32768 && outer_u * P.batch == 1;
+    if (inner == 1 && n <= row_max() && !lone) {
       PassRec* r = add();
       if (!r || !fft_pass(r, (int)n, 0, EPI_PLAIN, 0, 0, outer_u)) return;
       r->in = in;
@@ -578,7 +605,7 @@ struct Builder {
     // four-step along the axis: n = n1 * n2
     idx_t n2, n1;
     if (inner == 1) {
-      n2 = row_len_1d(n);
+      n2 = row_len_1d(n, few);
       if (P.mode != afft_gpu_mode_fma && n == 65536 && P.var.row_log2 <= 0) n2 = 256;  // 256 x 256 on the matrix cores
       if (n2 < 2 || n2 > 4096 || n2 >= n || !find_pass<T>((int)n2, 0, 0, EPI_PLAIN, 1)) {
         set_err("transform length %lld is too long", (long long)n);
@@ -612,7 +639,7 @@ struct Builder {
     }
     // pass A: length-n1 columns (stride n2*inner), twiddle W_n^(n2idx*k1)
     PassRec* a = add();
-    if (!a || !fft_pass(a, (int)n1, 1, EPI_TW4, 0)) return;
+    if (!a || !fft_pass(a, (int)n1, 1, EPI_TW4, 0, 0, 1, few)) return;
     a->in = in;
     a->out = tA;
     a->in.s_j = n2 * inner;
@@ -632,7 +659,7 @@ struct Builder {
     // pass B: length-n2 transforms of every (k1, c); output bin k1 + n1*k2
     PassRec* b = add();
     if (inner == 1) {
-      if (!b || !fft_pass(b, (int)n2, 0, EPI_PLAIN, 1)) return;
+      if (!b || !fft_pass(b, (int)n2, 0, EPI_PLAIN, 1, 0, 1, few)) return;
       b->in = tB;
       b->out = out;
       b->in.s_j = 1;
@@ -881,7 +908,11 @@ struct Builder {
     int cta = 0, sva = 0, hxa = 0, ctb = 0, svb = 0, hxb = 0;
     const int want_sv = P.var.sched < 0 ? 0 : (P.var.sched > 0 ? 1 : -1);
     const int want_hx = P.var.half_lds < 0 ? 0 : (P.var.half_lds > 0 ? 1 : -1);
-    if (!real4_shape(0, (int)sizeof(T), (int)std::min<idx_t>(n1, 1 << 30), P.var.col_tile, want_sv, want_hx, cta, sva,
+    // 2048-point columns, 16 per group, of a transform or two are fewer groups
+    // than CUs: 8 per group (2^22 x 1 56.1 -> 46.4 us, x 2 66.6 -> 62.8, x 4
+    // 88.8 -> 97.6; 2^23 x 1 69.1 -> 65.7, x 2 102.9 -> 108.7)
+    const bool narrow = n1 == 2048 && P.var.col_tile == 0 && P.var.real_pair == 0 && P.batch * N <= ((idx_t)1 << 23);
+    if (!real4_shape(0, (int)sizeof(T), (int)std::min<idx_t>(n1, 1 << 30), narrow ? 8 : P.var.col_tile, want_sv, want_hx, cta, sva,
                      hxa) ||
         !real4_shape(1, (int)sizeof(T), (int)std::min<idx_t>(n2, 1 << 30), P.var.rowt_tile, want_sv, want_hx, ctb,
                      svb, hxb) ||
@@ -958,7 +989,13 @@ struct Builder {
     int ctc = 0, svc = 0, hxc = 0, ctd = 0, svd = 0, hxd = 0;
     const int want_sv = P.var.sched < 0 ? 0 : (P.var.sched > 0 ? 1 : -1);
     const int want_hx = P.var.half_lds < 0 ? 0 : (P.var.half_lds > 0 ? 1 : -1);
-    if (!real4_shape(2, (int)sizeof(T), (int)std::min<idx_t>(n2, 1 << 30), P.var.col_tile, want_sv, want_hx, ctc, svc,
+    // the spectrum pass of few points: radix 16 (2^19 x 1 31.4 -> 25.0 us, x 4
+    // 30.3 -> 28.5; 2^20 x 1 27.4 -> 26.3, x 4 36.6 -> 34.2; 2^21 x 1 33.6 -> 29.3,
+    // x 2 39.4 -> 35.1, x 4 49.7 -> 50.9; 2^22 x 1 39.4 -> 35.8, x 2 50.6 -> 51.8)
+    const bool few = P.var.real_pair == 0 && few_points(N * P.batch, 22);
+    const int col_tile = few && P.var.col_tile == 0 && n2 == 1024 ? 16 : P.var.col_tile;
+    if (!real4_shape(2, (int)sizeof(T), (int)std::min<idx_t>(n2, 1 << 30), col_tile, few ? 0 : want_sv,
+                     few ? (n2 >= 1024 ? 0 : 1) : want_hx, ctc, svc,
                      hxc) ||
         !real4_shape(3, (int)sizeof(T), (int)std::min<idx_t>(n1, 1 << 30), P.var.rowt_tile, want_sv, want_hx, ctd,
                      svd, hxd) ||

@@ -475,7 +475,7 @@ struct R4Shape {
 // c2r spectrum pass: 8 columns per group at 1024 and 2048 points (64 x 2^20
 // 0.237 -> 0.207 ms, 16 x 2^22 0.254 -> 0.228 ms against 16 columns)
 #define AFGPU_R4C_SHAPES(X)                                                                                 \
-  X(256, 16, 0, 1) X(512, 16, 1, 1) X(1024, 8, 1, 1) X(1024, 16, 1, 1) X(1024, 16, 0, 0) X(2048, 8, 1, 1)   \
+  X(256, 16, 0, 1) X(512, 16, 1, 1) X(512, 16, 0, 1) X(1024, 8, 1, 1) X(1024, 16, 1, 1) X(1024, 16, 0, 0) X(2048, 8, 1, 1)   \
   X(2048, 16, 1, 1) X(2048, 8, 0, 0) X(4096, 4, 0, 1)
 #define AFGPU_R4D_SHAPES(X)                                                                                 \
   X(128, 16, 0, 1) X(256, 16, 0, 1) X(512, 16, 0, 1) X(1024, 8, 0, 1) X(1024, 16, 0, 0) X(1024, 16, 1, 1)  \
