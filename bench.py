@@ -224,7 +224,7 @@ def bench_mfma(torch, dev, stream, g, iters=5):
 
 def bench_queue(torch, dev, stream, reps=40):
     """10,000 1-D FP32 jobs, N = 2^k with k ~ U{6..16}, 70% complex / 30%
-    real, direction at random, in one persistent launch per batch; timed
+    real, direction at random, in one queue launch per batch; timed
     eagerly and as a replayed HIP graph (per-batch latency p50/p99)."""
     from fft_amd.afft import Queue
     rng = np.random.default_rng(5)

@@ -319,59 +319,61 @@ struct PassShape {
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
+// off: byte offset of the lane, checked against the extent; soff: a further offset
+// common to the wave (a scalar register), not checked.
 template <typename T, int AUX>
-__device__ __forceinline__ cx<T> buf_ld(__amdgpu_buffer_rsrc_t r, unsigned off);
+__device__ __forceinline__ cx<T> buf_ld(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff = 0);
 template <>
-__device__ __forceinline__ cx<float> buf_ld<float, 0>(__amdgpu_buffer_rsrc_t r, unsigned off) {
-  u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+__device__ __forceinline__ cx<float> buf_ld<float, 0>(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff) {
+  u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0);
   return {__uint_as_float(w.x), __uint_as_float(w.y)};
 }
 template <>
-__device__ __forceinline__ cx<float> buf_ld<float, 2>(__amdgpu_buffer_rsrc_t r, unsigned off) {
-  u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 2);
+__device__ __forceinline__ cx<float> buf_ld<float, 2>(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff) {
+  u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 2);
   return {__uint_as_float(w.x), __uint_as_float(w.y)};
 }
 template <>
-__device__ __forceinline__ cx<double> buf_ld<double, 0>(__amdgpu_buffer_rsrc_t r, unsigned off) {
-  u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+__device__ __forceinline__ cx<double> buf_ld<double, 0>(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff) {
+  u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0);
   return {__hiloint2double(w.y, w.x), __hiloint2double(w.w, w.z)};
 }
 template <>
-__device__ __forceinline__ cx<double> buf_ld<double, 2>(__amdgpu_buffer_rsrc_t r, unsigned off) {
-  u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 2);
+__device__ __forceinline__ cx<double> buf_ld<double, 2>(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff) {
+  u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 2);
   return {__hiloint2double(w.y, w.x), __hiloint2double(w.w, w.z)};
 }
 template <int AUX>
-__device__ __forceinline__ void buf_st(cx<float> v, __amdgpu_buffer_rsrc_t r, unsigned off) {
+__device__ __forceinline__ void buf_st(cx<float> v, __amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff = 0) {
   u32x2 w = {__float_as_uint(v.x), __float_as_uint(v.y)};
-  __builtin_amdgcn_raw_buffer_store_b64(w, r, off, 0, AUX);
+  __builtin_amdgcn_raw_buffer_store_b64(w, r, off, soff, AUX);
 }
 template <int AUX>
-__device__ __forceinline__ void buf_st(cx<double> v, __amdgpu_buffer_rsrc_t r, unsigned off) {
+__device__ __forceinline__ void buf_st(cx<double> v, __amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff = 0) {
   unsigned long long a = __double_as_longlong(v.x), b = __double_as_longlong(v.y);
   u32x4 w = {(unsigned)a, (unsigned)(a >> 32), (unsigned)b, (unsigned)(b >> 32)};
-  __builtin_amdgcn_raw_buffer_store_b128(w, r, off, 0, AUX);
+  __builtin_amdgcn_raw_buffer_store_b128(w, r, off, soff, AUX);
 }
 
 // one part (real or imaginary) of an element
 template <typename T, int AUX>
-__device__ __forceinline__ T buf_ld1(__amdgpu_buffer_rsrc_t r, unsigned off) {
+__device__ __forceinline__ T buf_ld1(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff = 0) {
   if constexpr (std::is_same_v<T, float>) {
-    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, AUX));
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, soff, AUX));
   } else {
-    u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, AUX);
+    u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, AUX);
     return __hiloint2double(w.y, w.x);
   }
 }
 template <int AUX>
-__device__ __forceinline__ void buf_st1(float v, __amdgpu_buffer_rsrc_t r, unsigned off) {
-  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, off, 0, AUX);
+__device__ __forceinline__ void buf_st1(float v, __amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff = 0) {
+  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, off, soff, AUX);
 }
 template <int AUX>
-__device__ __forceinline__ void buf_st1(double v, __amdgpu_buffer_rsrc_t r, unsigned off) {
+__device__ __forceinline__ void buf_st1(double v, __amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff = 0) {
   unsigned long long a = __double_as_longlong(v);
   u32x2 w = {(unsigned)a, (unsigned)(a >> 32)};
-  __builtin_amdgcn_raw_buffer_store_b64(w, r, off, 0, AUX);
+  __builtin_amdgcn_raw_buffer_store_b64(w, r, off, soff, AUX);
 }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, unsigned bytes) {

@@ -45,6 +45,71 @@ __device__ __forceinline__ cx<T> real4_tw(const Real4Args<T>& a, unsigned mask, 
   return tw4_lookup32(a.tw4_hi, a.tw4_lo, a.tw4_bits, mask, e);
 }
 
+// Passes B' and, but for 1024-point rows, B (and the 2048-point pass A) read and write through buffer
+// resources, one per array and transform (at most 2^23 reals, so 32-bit byte
+// offsets), with the format and cache policy chosen once per phase.  As 64-bit
+// addresses with a branch on both around each access B' took 88.2 us per 134 MB
+// at 2048 points (71.0 now), 89.5 at 1024 (75.6), and B 92.0 at 2048
+// (85.5).  Pass A' gained nothing and keeps its addresses.
+template <typename F>
+__device__ __forceinline__ void r4_policy(bool split, bool nt, F&& f) {
+  if (split) {
+    if (nt)
+      f(std::integral_constant<int, POL_SPLIT | POL_NT>{});
+    else
+      f(std::integral_constant<int, POL_SPLIT>{});
+  } else {
+    if (nt)
+      f(std::integral_constant<int, POL_NT>{});
+    else
+      f(std::integral_constant<int, 0>{});
+  }
+}
+// A complex array of one transform: n elements at element offset `base`.
+struct R4Side {
+  __amdgpu_buffer_rsrc_t re, im;
+};
+template <typename T>
+__device__ __forceinline__ R4Side r4_side(const T* re, const T* im, bool split, idx_t base, idx_t n) {
+  if (split) return {make_rsrc(re + base, (unsigned)(n * sizeof(T))), make_rsrc(im + base, (unsigned)(n * sizeof(T)))};
+  const __amdgpu_buffer_rsrc_t r = make_rsrc(reinterpret_cast<const cx<T>*>(re) + base, (unsigned)(n * sizeof(cx<T>)));
+  return {r, r};
+}
+// Element e + s: e per lane (an e past the array reads zero and drops stores
+// whatever s is), s common to the wave.  Split like this a tile's accesses share
+// one address register.
+template <typename T, int POL>
+__device__ __forceinline__ cx<T> r4_ld(const R4Side& a, unsigned e, unsigned s) {
+  constexpr unsigned ES = sizeof(cx<T>), ET = sizeof(T);
+  if constexpr (POL & POL_SPLIT)
+    return {buf_ld1<T, POL & POL_NT>(a.re, e * ET, s * ET), buf_ld1<T, POL & POL_NT>(a.im, e * ET, s * ET)};
+  else
+    return buf_ld<T, POL & POL_NT>(a.re, e * ES, s * ES);
+}
+template <int POL, typename T>
+__device__ __forceinline__ void r4_st(const R4Side& a, unsigned e, unsigned s, cx<T> z) {
+  constexpr unsigned ES = sizeof(cx<T>), ET = sizeof(T);
+  if constexpr (POL & POL_SPLIT) {
+    buf_st1<POL & POL_NT>(z.x, a.re, e * ET, s * ET);
+    buf_st1<POL & POL_NT>(z.y, a.im, e * ET, s * ET);
+  } else {
+    buf_st<POL & POL_NT>(z, a.re, e * ES, s * ES);
+  }
+}
+
+// Elements e + s and e + s + 1 of an interleaved array (FP32: in one access; as
+// two, the 2048-point pass A took 72.8 us instead of 68.5).
+template <typename T>
+__device__ __forceinline__ void r4_st2(const R4Side& a, unsigned e, unsigned s, cx<T> z0, cx<T> z1) {
+  if constexpr (std::is_same_v<T, float>) {
+    const u32x4 w = {__float_as_uint(z0.x), __float_as_uint(z0.y), __float_as_uint(z1.x), __float_as_uint(z1.y)};
+    __builtin_amdgcn_raw_buffer_store_b128(w, a.re, e * 8u, s * 8u, 0);
+  } else {
+    r4_st<0>(a, e, s, z0);
+    r4_st<0>(a, e + 1, s, z1);
+  }
+}
+
 template <typename T, int L, int CT, int SV, bool HX>
 struct R4AShape {
   using PS = PassShape<L, CT, SV>;
@@ -89,12 +154,26 @@ __global__ void __launch_bounds__((R4AShape<T, L, CT, SV, HX>::NT), (R4AShape<T,
   auto latf = [&](int i) -> T& { return ldsf[lds_pad(i) * CT + c]; };
 
   // element j1 of packed column col: the reals x[j1*n2 + 2col], x[j1*n2 + 2col + 1]
-  const T* src = a.in + b * a.in_bs + 2 * col;
+  // (2048 points through buffers, shorter columns through 64-bit addresses: us per
+  // 134 MB of reals, addresses / buffers, 2048 72.5 / 68.5, 1024 55.7 / 61.9, 512
+  // 56.7 / 55.8)
+  constexpr bool BUF = L >= 2048;
   cx<T> v[E];
-  static_for<E>([&](auto mc) AFGPU_INLINE {
-    constexpr int m = decltype(mc)::value;
-    v[m] = ld_elem<T>(src, nullptr, 1, (idx_t)(t + m * TPT) * npc, a.in_nt);
-  });
+  if constexpr (BUF) {
+    const R4Side src = r4_side<T>(a.in + b * a.in_bs, nullptr, false, 0, a.n1 * npc);
+    r4_policy(false, a.in_nt, [&](auto pol) AFGPU_INLINE {
+      static_for<E>([&](auto mc) AFGPU_INLINE {
+        constexpr int m = decltype(mc)::value;
+        v[m] = r4_ld<T, decltype(pol)::value>(src, (unsigned)t * (unsigned)npc + (unsigned)col, m * TPT * (unsigned)npc);
+      });
+    });
+  } else {
+    const T* src = a.in + b * a.in_bs + 2 * col;
+    static_for<E>([&](auto mc) AFGPU_INLINE {
+      constexpr int m = decltype(mc)::value;
+      v[m] = ld_elem<T>(src, nullptr, 1, (idx_t)(t + m * TPT) * npc, a.in_nt);
+    });
+  }
   if constexpr (HX)
     run_stages<T, L, SV, 0, true, CT>(v, t, latf, a.stage_tw);
   else
@@ -128,7 +207,8 @@ __global__ void __launch_bounds__((R4AShape<T, L, CT, SV, HX>::NT), (R4AShape<T,
 
   // unpack, twiddle, store rows k1 <= n1/2 of Y (columns 2col, 2col + 1)
   const unsigned mask = (1u << a.tw4_bits) - 1u;
-  cx<T>* dst = a.scr + b * a.scr_bs + 2 * col;
+  const R4Side dst = r4_side<T>(reinterpret_cast<const T*>(a.scr), nullptr, false, b * a.scr_bs, (a.n1 / 2 + 1) * a.n2);
+  cx<T>* dst_row = a.scr + b * a.scr_bs + 2 * col;
   const T h = T(0.5);
   static_for<MH + 1>([&](auto mc) AFGPU_INLINE {
     constexpr int m = decltype(mc)::value;
@@ -141,9 +221,13 @@ __global__ void __launch_bounds__((R4AShape<T, L, CT, SV, HX>::NT), (R4AShape<T,
       const unsigned e0 = (unsigned)(2 * col) * (unsigned)k1;
       A = cmul(A, real4_tw(a, mask, e0));
       B = cmul(B, real4_tw(a, mask, e0 + (unsigned)k1));
-      cx<T>* row = dst + (idx_t)k1 * a.n2;
-      row[0] = A;
-      row[1] = B;
+      if constexpr (BUF) {
+        r4_st2(dst, (unsigned)t * (unsigned)a.n2 + 2 * (unsigned)col, m * TPT * (unsigned)a.n2, A, B);
+      } else {
+        cx<T>* row = dst_row + (idx_t)k1 * a.n2;
+        row[0] = A;
+        row[1] = B;
+      }
     }
   });
 }
@@ -165,7 +249,7 @@ __global__ void __launch_bounds__((R4BShape<T, L, CT, SV, HX>::NT), (R4BShape<T,
   constexpr int E = S::E;
   constexpr int TPT = S::TPT;
   constexpr int LL = S::LL;
-  constexpr int MH = E / 2;  // registers m <= MH of the store phase hold bins k2 <= L/2
+  constexpr int MH = E / 2;  // registers m < MH of the store phase hold bins k2 < L/2
   extern __shared__ __align__(16) unsigned char afgpu_smem[];
   cx<T>* __restrict__ lds = reinterpret_cast<cx<T>*>(afgpu_smem);
   T* __restrict__ ldsf = reinterpret_cast<T*>(afgpu_smem);
@@ -182,11 +266,24 @@ __global__ void __launch_bounds__((R4BShape<T, L, CT, SV, HX>::NT), (R4BShape<T,
   auto latf = [&](int i) -> T& { return ldsf[c * LL + lds_pad(i)]; };
 
   cx<T> v[E];
-  const cx<T>* src = a.scr + b * a.scr_bs + row * a.n2;
-  static_for<E>([&](auto mc) AFGPU_INLINE {
-    constexpr int m = decltype(mc)::value;
-    v[m] = row < nrows ? src[t + m * TPT] : cx<T>{T(0), T(0)};
-  });
+  // 1024-point rows keep 64-bit addresses and a condition on each store: us per
+  // 1 GiB of reals, so / through buffers, 2^19 x 512 1098 / 1143, 2^20 x 256 1117
+  // / 1150 (2^16 x 4096, 256-point rows, 1081 / 1015; 256 MiB, 2^22 x 16, 2048, 321 / 300)
+  constexpr bool BUF = L != 1024;
+  if constexpr (BUF) {
+    // (rows past the last lie beyond the extent and read as zero)
+    const R4Side src = r4_side<T>(reinterpret_cast<const T*>(a.scr), nullptr, false, b * a.scr_bs, nrows * a.n2);
+    static_for<E>([&](auto mc) AFGPU_INLINE {
+      constexpr int m = decltype(mc)::value;
+      v[m] = r4_ld<T, 0>(src, (unsigned)row * (unsigned)a.n2 + (unsigned)t, m * TPT);
+    });
+  } else {
+    const cx<T>* src = a.scr + b * a.scr_bs + row * a.n2;
+    static_for<E>([&](auto mc) AFGPU_INLINE {
+      constexpr int m = decltype(mc)::value;
+      v[m] = row < nrows ? src[t + m * TPT] : cx<T>{T(0), T(0)};
+    });
+  }
   if constexpr (HX)
     run_stages<T, L, SV, 0, true, 1>(v, t, latf, a.stage_tw);
   else
@@ -195,44 +292,94 @@ __global__ void __launch_bounds__((R4BShape<T, L, CT, SV, HX>::NT), (R4BShape<T,
   // store phase: lane c2 = tid % CT takes row row0 + c2, bins k2 = t2 + m*TPT
   const int c2 = tid % CT, t2 = tid / CT;
   const idx_t r2 = row0 + c2;
-  const idx_t n1 = a.n1;
-  const idx_t ob = b * a.out_bs;
-  auto own = [&](int k2) AFGPU_INLINE { return r2 <= half && (k2 < L / 2 || (r2 == 0 && k2 == L / 2)); };
-  auto mirror = [&](int k2) AFGPU_INLINE { return r2 > 0 && r2 < half && k2 < L / 2; };
+  if constexpr (!BUF) {
+    const idx_t n1 = a.n1;
+    const idx_t ob = b * a.out_bs;
+    auto own = [&](int k2) AFGPU_INLINE { return r2 <= half && (k2 < L / 2 || (r2 == 0 && k2 == L / 2)); };
+    auto mirror = [&](int k2) AFGPU_INLINE { return r2 > 0 && r2 < half && k2 < L / 2; };
+    if constexpr (!HX) {
+      static_for<E>([&](auto mc) AFGPU_INLINE { lat(t + decltype(mc)::value * TPT) = v[decltype(mc)::value]; });
+      __syncthreads();
+      static_for<MH + 1>([&](auto mc) AFGPU_INLINE {
+        constexpr int m = decltype(mc)::value;
+        const int k2 = t2 + m * TPT;
+        if (own(k2)) r4_store(a, ob + r2 + n1 * k2, lds[c2 * LL + lds_pad(k2)]);
+        if (mirror(k2)) r4_store(a, ob + (n1 - r2) + n1 * k2, conjg(lds[c2 * LL + lds_pad(L - 1 - k2)]));
+      });
+    } else {
+      T xo[MH + 1], xm[MH + 1];
+      static_for<E>([&](auto mc) AFGPU_INLINE { latf(t + decltype(mc)::value * TPT) = v[decltype(mc)::value].x; });
+      __syncthreads();
+      static_for<MH + 1>([&](auto mc) AFGPU_INLINE {
+        constexpr int m = decltype(mc)::value;
+        const int k2 = t2 + m * TPT;
+        xo[m] = ldsf[c2 * LL + lds_pad(k2)];
+        xm[m] = ldsf[c2 * LL + lds_pad(L - 1 - k2)];
+      });
+      __syncthreads();
+      static_for<E>([&](auto mc) AFGPU_INLINE { latf(t + decltype(mc)::value * TPT) = v[decltype(mc)::value].y; });
+      __syncthreads();
+      static_for<MH + 1>([&](auto mc) AFGPU_INLINE {
+        constexpr int m = decltype(mc)::value;
+        const int k2 = t2 + m * TPT;
+        if (own(k2)) r4_store(a, ob + r2 + n1 * k2, cx<T>{xo[m], ldsf[c2 * LL + lds_pad(k2)]});
+        if (mirror(k2)) r4_store(a, ob + (n1 - r2) + n1 * k2, cx<T>{xm[m], -ldsf[c2 * LL + lds_pad(L - 1 - k2)]});
+      });
+    }
+    return;
+  }
+  const unsigned n1 = (unsigned)a.n1;
+  const R4Side dst = r4_side<T>(a.out_re, a.out_im, !a.out_il, b * a.out_bs, a.n1 * a.n2 / 2 + 1);
+  // Registers m < E/2 hold k2 = t2 + m*TPT < n2/2: bins of the own row go to
+  // r2 + n1*k2, of the mirrored one to n1 - r2 + n1*k2; a row past the last, or without a mirror
+  // (rows 0 and n1/2), has its offsets beyond the extent, where stores are
+  // dropped, so no store carries a condition.  Bin N/2 is row 0's k2 = n2/2.
+  constexpr unsigned kNone = 1u << 27;
+  const unsigned o0 = (r2 <= half ? (unsigned)r2 : kNone) + n1 * (unsigned)t2;
+  const unsigned m0 = (r2 > 0 && r2 < half ? n1 - (unsigned)r2 : kNone) + n1 * (unsigned)t2;
+  const bool last = r2 == 0 && t2 == 0;
+  // LDS entries as one address each plus constants (TPT is a multiple of 16):
+  // of row c, entry t + m*TPT at pt + m*step; of row c2, entry k2 at po + m*step
+  // and L - 1 - k2 at pm + (MH - 1 - m)*step
+  constexpr int step = pad_step<TPT>();
+  static_assert(step > 0, "padded indices of a tile's entries are affine in m");
+  const int pt = c * LL + lds_pad(t), po = c2 * LL + lds_pad(t2);
+  const int pm = c2 * LL + lds_pad(L - 1 - t2) - (MH - 1) * step;
   if constexpr (!HX) {
-    static_for<E>([&](auto mc) AFGPU_INLINE { lat(t + decltype(mc)::value * TPT) = v[decltype(mc)::value]; });
+    static_for<E>([&](auto mc) AFGPU_INLINE { lds[pt + decltype(mc)::value * step] = v[decltype(mc)::value]; });
     __syncthreads();
-    static_for<MH + 1>([&](auto mc) AFGPU_INLINE {
-      constexpr int m = decltype(mc)::value;
-      const int k2 = t2 + m * TPT;
-      if (own(k2)) r4_store(a, ob + r2 + n1 * k2, lds[c2 * LL + lds_pad(k2)]);
-      if (mirror(k2)) r4_store(a, ob + (n1 - r2) + n1 * k2, conjg(lds[c2 * LL + lds_pad(L - 1 - k2)]));
+    r4_policy(!a.out_il, a.out_nt, [&](auto polc) AFGPU_INLINE {
+      constexpr int pol = decltype(polc)::value;
+      static_for<MH>([&](auto mc) AFGPU_INLINE {
+        constexpr int m = decltype(mc)::value;
+        r4_st<pol>(dst, o0, n1 * (m * TPT), lds[po + m * step]);
+        r4_st<pol>(dst, m0, n1 * (m * TPT), conjg(lds[pm + (MH - 1 - m) * step]));
+      });
+      if (last) r4_st<pol>(dst, n1 * (unsigned)(L / 2), 0, lds[c2 * LL + lds_pad(L / 2)]);
     });
   } else {
-    T xo[MH + 1], xm[MH + 1];
-    static_for<E>([&](auto mc) AFGPU_INLINE { latf(t + decltype(mc)::value * TPT) = v[decltype(mc)::value].x; });
+    T xo[MH], xm[MH];
+    static_for<E>([&](auto mc) AFGPU_INLINE { ldsf[pt + decltype(mc)::value * step] = v[decltype(mc)::value].x; });
     __syncthreads();
-    static_for<MH + 1>([&](auto mc) AFGPU_INLINE {
+    static_for<MH>([&](auto mc) AFGPU_INLINE {
       constexpr int m = decltype(mc)::value;
-      const int k2 = t2 + m * TPT;
-      xo[m] = ldsf[c2 * LL + lds_pad(k2)];
-      xm[m] = ldsf[c2 * LL + lds_pad(L - 1 - k2)];
+      xo[m] = ldsf[po + m * step];
+      xm[m] = ldsf[pm + (MH - 1 - m) * step];
     });
+    const T xl = last ? ldsf[c2 * LL + lds_pad(L / 2)] : T(0);
     __syncthreads();
-    static_for<E>([&](auto mc) AFGPU_INLINE { latf(t + decltype(mc)::value * TPT) = v[decltype(mc)::value].y; });
+    static_for<E>([&](auto mc) AFGPU_INLINE { ldsf[pt + decltype(mc)::value * step] = v[decltype(mc)::value].y; });
     __syncthreads();
-    static_for<MH + 1>([&](auto mc) AFGPU_INLINE {
-      constexpr int m = decltype(mc)::value;
-      const int k2 = t2 + m * TPT;
-      if (own(k2)) r4_store(a, ob + r2 + n1 * k2, cx<T>{xo[m], ldsf[c2 * LL + lds_pad(k2)]});
-      if (mirror(k2)) r4_store(a, ob + (n1 - r2) + n1 * k2, cx<T>{xm[m], -ldsf[c2 * LL + lds_pad(L - 1 - k2)]});
+    r4_policy(!a.out_il, a.out_nt, [&](auto polc) AFGPU_INLINE {
+      constexpr int pol = decltype(polc)::value;
+      static_for<MH>([&](auto mc) AFGPU_INLINE {
+        constexpr int m = decltype(mc)::value;
+        r4_st<pol>(dst, o0, n1 * (m * TPT), cx<T>{xo[m], ldsf[po + m * step]});
+        r4_st<pol>(dst, m0, n1 * (m * TPT), cx<T>{xm[m], -ldsf[pm + (MH - 1 - m) * step]});
+      });
+      if (last) r4_st<pol>(dst, n1 * (unsigned)(L / 2), 0, cx<T>{xl, ldsf[c2 * LL + lds_pad(L / 2)]});
     });
   }
-}
-
-template <typename T>
-__device__ __forceinline__ cx<T> r4_load_in(const Real4Args<T>& a, idx_t e) {
-  return a.in_il ? ld_elem<T>(a.in, nullptr, 1, e, a.in_nt) : ld_elem<T>(a.in, a.in_im, 0, e, a.in_nt);
 }
 
 // c2r pass B': CT consecutive columns k1 of the spectrum viewed as n2 rows of
@@ -264,21 +411,24 @@ __global__ void __launch_bounds__((R4AShape<T, L, CT, SV, HX>::NT), (R4AShape<T,
   auto latf = [&](int i) -> T& { return ldsf[lds_pad(i) * CT + c]; };
 
   cx<T> v[E];
-  static_for<E>([&](auto mc) AFGPU_INLINE {
-    constexpr int m = decltype(mc)::value;
-    const int k2 = t + m * TPT;
-    cx<T> z = {T(0), T(0)};
-    if (live) {
-      if (m < E / 2 || (k1 == 0 && k2 == L / 2)) {
-        z = r4_load_in(a, ib + k1 + n1 * k2);
-        if (k1 == 0 && (k2 == 0 || k2 == L / 2)) z.y = T(0);  // bins 0 and N/2: real parts only
-      } else if (k1 == 0) {
-        z = conjg(r4_load_in(a, ib + n1 * (L - k2)));
-      } else {
-        z = conjg(r4_load_in(a, ib + (n1 - k1) + n1 * (L - 1 - k2)));
-      }
-    }
-    v[m] = swapri(z);  // inverse DFT as swap(DFT(swap(.)))
+  // own bins for k2 < n2/2, mirrored ones beyond: n1*(n2 - k2) - k1 is also
+  // right for column 0, and at k2 = n2/2 of column 0 both name bin N/2.  Dead
+  // columns read past the extent, which gives zero.
+  const idx_t nbins = n1 * a.n2 / 2 + 1;
+  const R4Side src = r4_side<T>(a.in, a.in_im, !a.in_il, ib, nbins);
+  const unsigned un1 = (unsigned)n1, uk1 = (unsigned)k1;
+  // k2 = t + m*TPT, n2 - k2 = (TPT - t) + (E - 1 - m)*TPT
+  const unsigned e_own = live ? uk1 + un1 * (unsigned)t : (unsigned)nbins;
+  const unsigned e_mir = live ? un1 * (unsigned)(TPT - t) - uk1 : (unsigned)nbins;
+  r4_policy(!a.in_il, a.in_nt, [&](auto polc) AFGPU_INLINE {
+    static_for<E>([&](auto mc) AFGPU_INLINE {
+      constexpr int m = decltype(mc)::value;
+      cx<T> z = m < E / 2 ? r4_ld<T, decltype(polc)::value>(src, e_own, un1 * (m * TPT))
+                          : r4_ld<T, decltype(polc)::value>(src, e_mir, un1 * ((E - 1 - m) * TPT));
+      if constexpr (m >= E / 2) z = conjg(z);
+      if ((m == 0 || m == E / 2) && k1 == 0 && t == 0) z.y = T(0);  // bins 0 and N/2: real parts only
+      v[m] = swapri(z);  // inverse DFT as swap(DFT(swap(.)))
+    });
   });
   if constexpr (HX)
     run_stages<T, L, SV, 0, true, CT>(v, t, latf, a.stage_tw);
@@ -286,12 +436,12 @@ __global__ void __launch_bounds__((R4AShape<T, L, CT, SV, HX>::NT), (R4AShape<T,
     run_stages<T, L, SV, 0, false, CT>(v, t, lat, a.stage_tw);
   if (live) {
     const unsigned mask = (1u << a.tw4_bits) - 1u;
-    cx<T>* dst = a.scr + b * a.scr_bs + k1;
+    const R4Side dst = r4_side<T>(reinterpret_cast<const T*>(a.scr), nullptr, false, b * a.scr_bs, a.n2 * a.rs);
     static_for<E>([&](auto mc) AFGPU_INLINE {
       constexpr int m = decltype(mc)::value;
       const int j2 = t + m * TPT;
       const cx<T> wt = real4_tw(a, mask, (unsigned)j2 * (unsigned)k1);
-      dst[(idx_t)j2 * a.rs] = cmulc(swapri(v[m]), wt);
+      r4_st<0>(dst, (unsigned)t * (unsigned)a.rs + uk1, m * TPT * (unsigned)a.rs, cmulc(swapri(v[m]), wt));
     });
   }
 }
