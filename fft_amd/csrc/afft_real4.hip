@@ -45,11 +45,11 @@ __device__ __forceinline__ cx<T> real4_tw(const Real4Args<T>& a, unsigned mask, 
   return tw4_lookup32(a.tw4_hi, a.tw4_lo, a.tw4_bits, mask, e);
 }
 
-// Passes B' and, but for 1024-point rows, B (and the 2048-point pass A) read and write through buffer
-// resources, one per array and transform (at most 2^23 reals, so 32-bit byte
-// offsets), with the format and cache policy chosen once per phase.  As 64-bit
-// addresses with a branch on both around each access B' took 88.2 us per 134 MB
-// at 2048 points (71.0 now), 89.5 at 1024 (75.6), and B 92.0 at 2048
+// Pass B', B (but for 1024-point rows) and the 2048-point pass A read and write
+// through buffer resources, one per array and transform (at most 2^23 reals, so
+// 32-bit byte offsets), with the format and cache policy chosen once per phase.
+// As 64-bit addresses with a branch on both around each access B' took 88.2 us
+// per 134 MB at 2048 points (71.0 now), 89.5 at 1024 (75.6), and B 92.0 at 2048
 // (85.5).  Pass A' gained nothing and keeps its addresses.
 template <typename F>
 __device__ __forceinline__ void r4_policy(bool split, bool nt, F&& f) {
@@ -331,9 +331,10 @@ __global__ void __launch_bounds__((R4BShape<T, L, CT, SV, HX>::NT), (R4BShape<T,
   const unsigned n1 = (unsigned)a.n1;
   const R4Side dst = r4_side<T>(a.out_re, a.out_im, !a.out_il, b * a.out_bs, a.n1 * a.n2 / 2 + 1);
   // Registers m < E/2 hold k2 = t2 + m*TPT < n2/2: bins of the own row go to
-  // r2 + n1*k2, of the mirrored one to n1 - r2 + n1*k2; a row past the last, or without a mirror
-  // (rows 0 and n1/2), has its offsets beyond the extent, where stores are
-  // dropped, so no store carries a condition.  Bin N/2 is row 0's k2 = n2/2.
+  // r2 + n1*k2, of the mirrored one to n1 - r2 + n1*k2; a row past the last, or
+  // without a mirror (rows 0 and n1/2), has its offsets beyond the extent, where
+  // stores are dropped, so no store carries a condition.  Bin N/2 is row 0's
+  // k2 = n2/2.
   constexpr unsigned kNone = 1u << 27;
   const unsigned o0 = (r2 <= half ? (unsigned)r2 : kNone) + n1 * (unsigned)t2;
   const unsigned m0 = (r2 > 0 && r2 < half ? n1 - (unsigned)r2 : kNone) + n1 * (unsigned)t2;
