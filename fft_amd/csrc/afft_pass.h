@@ -799,16 +799,18 @@ constexpr size_t tile_lds_bytes() {
 
 // Minimum waves per SIMD the compiler must allow for: half-exchange tiles
 // that fit twice in a CU's 160 KiB of LDS are meant to run two groups per CU,
-// so their registers are bounded accordingly; everything else runs one.
-
+// so their registers are bounded accordingly; everything else runs one.  Single
+// rows of 32 elements a thread in 256 threads (8192 points, FP32) are meant to
+// run four.  Rows of 16 elements a thread stay at two: with the bound of four
+// the FP64 4096-point ones spilled 10 VGPRs (512 MiB per side: c2c 4096 x 8192
+// 199.7 us, 186.8 at two; c2r 8192 x 8192 271, 235).
 template <typename T, int L, int CT, bool COLMAP, bool STORE_T, int SV, bool HX>
 constexpr int pass_min_waves() {
-  constexpr int nt = PassShape<L, CT, SV>::NT;
+  using PS = PassShape<L, CT, SV>;
   constexpr size_t lds = tile_lds_bytes<T, L, CT, COLMAP, STORE_T, SV, HX>();
-  // 256-thread rows of 32 elements a thread (8192 points): four groups per CU
-  if (HX && nt == 256 && 4 * lds <= 160 * 1024) return 4;
-  constexpr int groups = (HX && 2 * tile_lds_bytes<T, L, CT, COLMAP, STORE_T, SV, HX>() <= 160 * 1024) ? 2 : 1;
-  return groups * nt / 256 > 1 ? groups * nt / 256 : 1;
+  constexpr bool four = HX && CT == 1 && PS::E == 32 && PS::NT == 256 && 4 * lds <= 160 * 1024;
+  constexpr int groups = four ? 4 : (HX && 2 * lds <= 160 * 1024) ? 2 : 1;
+  return groups * PS::NT / 256 > 1 ? groups * PS::NT / 256 : 1;
 }
 
 template <typename T, int L, int CT, bool COLMAP, int EPI, bool STORE_T, int MODE, int SV, bool HX>
