@@ -188,6 +188,10 @@ struct Plan {
   // both passes of a 1-D FP32 c2c four-step in one persistent launch
   // (afft_fused.hip): ring slots per XCD and the pass-B lag, 0 = off
   int fused_slots = 0, fused_lag = 0;
+  // a lone 32768-point transform: the one-row pass that calls in place run
+  // instead of the pass list (lone_passes)
+  bool has_in_place = false;
+  PassRec in_place;
 };
 
 // Plans sit at the first kPlanAlign boundary of `mem` (any alignment accepted,
@@ -543,10 +547,7 @@ struct Builder {
     const int tmp_role = (in.role == R_SCR || out.role == R_SCR) ? R_SCR2 : R_SCR;
 
     const bool few = inner == 1 && few_points(n * outer_u * P.batch, n >= ((idx_t)1 << 20) ? 22 : 21);
-    // a single 32768-point transform: one group of one CU takes 25 us, the
-    // four-step over 64 groups 14
-    const bool lone = few && n == 32768 && outer_u * P.batch == 1;
-    if (inner == 1 && n <= row_max() && !lone) {
+    if (inner == 1 && n <= row_max()) {
       PassRec* r = add();
       if (!r || !fft_pass(r, (int)n, 0, EPI_PLAIN, 0, 0, outer_u)) return;
       r->in = in;
@@ -566,6 +567,7 @@ struct Builder {
       r->swap_in = swi;
       r->swap_out = swo;
       tiny(r);
+      if (few && n == 32768 && P.ndim == 1 && P.kind <= 1 && P.batch == 1) lone_passes(in, out, n, swi, swo);
       return;
     }
     // batch stride of a side whose batch index runs over (user, outer)
@@ -694,6 +696,49 @@ struct Builder {
       b->n_blo = (int)n1;
       b->b_per_user = outer_u * n1;
     }
+    b->swap_out = swo;
+  }
+
+  // A single 32768-point transform: one row is one group on one CU, 25.6 us (split
+  // 27.8); as 64 x 512 over 32 and 8 groups 11.0 (12.9).  It keeps the row's independence of
+  // everything but its own buffers (no scratch, so it can be captured at its
+  // first call and run beside any other call): pass A writes the output array,
+  // bin k1 of column j at k1 + 64 j, and pass B works in place there, on the 512
+  // entries k1 + 64 j of row k1, which are also where its bins k1 + 64 k2 go.  A
+  // call in place, where pass A would overwrite input that other groups have
+  // yet to read, runs the row.
+  void lone_passes(const Side& in, const Side& out, idx_t n, int swi, int swo) {
+    P.in_place = P.pass[--P.npass];
+    P.has_in_place = true;
+    const idx_t n2 = row_len_1d(n, true), n1 = n / n2;
+    const int bits = (ilog2(n) + 1) / 2;
+    const void* tw4 = get_table<T>(1, n, bits);
+    PassRec* a = add();
+    if (!tw4 || !a || !fft_pass(a, (int)n1, 1, EPI_TW4, 0, 0, 1, true)) {
+      ok = false;
+      return;
+    }
+    a->in = in;
+    a->out = out;
+    a->in.s_j = n2;
+    a->in.s_c = 1;
+    a->out.s_j = 1;
+    a->out.s_c = n1;
+    a->in.s_b = a->out.s_b = n;
+    a->n_col = n2;
+    a->swap_in = swi;
+    a->tw4_hi = tw4;
+    a->tw4_lo = (const cx<T>*)tw4 + (n >> bits);
+    a->tw4_n = n;
+    a->tw4_bits = bits;
+    PassRec* b = add();
+    if (!b || !fft_pass(b, (int)n2, 0, EPI_PLAIN, 1, 0, 1, true)) return;
+    b->in = out;
+    b->out = out;
+    b->in.s_j = b->out.s_j = n1;
+    b->in.s_c = b->out.s_c = 1;
+    b->in.s_b = b->out.s_b = n;
+    b->n_col = n1;
     b->swap_out = swo;
   }
 
@@ -1285,6 +1330,7 @@ struct Builder {
 
   bool build(int kind, int format, const idx_t* d, int nd) {
     P.npass = 0;
+    P.has_in_place = false;
     P.scr_per_user[0] = P.scr_per_user[1] = 0;
     bool r = build_passes(kind, format, d, nd);
     // stream_io 2: an N-D plan (its outer axes re-read dst) whose arrays hold at
@@ -1334,6 +1380,10 @@ struct Builder {
         q.mfma_mats = get_table<T>(3, 256, P.mode == afft_gpu_mode_mfma_bf16 ? 1 : 0);
         if (!q.mfma_mats) ok = false;
       }
+    }
+    if (P.has_in_place) {
+      P.in_place.in_nt = P.in_place.out_nt = P.var.stream_io != 0;
+      P.in_place.xcd = P.var.xcd_order;
     }
     if (r && ok && P.var.tiny_rows > 0 && P.var.tiny_rows != 64 && P.var.tiny_rows != 128 &&
         P.var.tiny_rows != 256) {
@@ -2110,6 +2160,8 @@ bool execute_on(Plan& P, const void* sre, const void* sim, void* dre, void* dim,
     B.src_im = nullptr;
     B.dst_im = nullptr;
   }
+  if (P.has_in_place && sre == dre && (P.format == afft_interleaved || sim == dim))
+    return first >= last || last < P.npass || run_pass<T>(P.in_place, B, 0, 1, st);
   if (P.fused_slots && !plain && first == 0 && last == P.npass) {
     // both passes in one persistent launch over the whole batch
     const PassRec& a = P.pass[0];
@@ -2186,7 +2238,8 @@ bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
 
 // Buffers may overlap: complex transforms run exactly in place (src == dst:
 // every pass reads a tile completely before it writes the same tile, and the
-// four-step passes go through scratch); any other overlap of input and output
+// four-step passes go through scratch or have a one-row form for such calls);
+// any other overlap of input and output
 // (real transforms in place, shifted buffers) first copies the input into
 // scratch and runs from there.  Staging says how many input arrays to copy
 // (0 = none) and their size.

@@ -76,7 +76,9 @@ int afft_gpu_execute_noalloc(afft_gpu_plan* plan, const void* src_re, const void
 
 /* Enqueues only passes [first, last) of the plan (last = -1: to the end),
  * for every chunk of the batch.  For measuring one kernel of a multi-pass
- * plan; running the ranges in order equals afft_gpu_execute. */
+ * plan; running the ranges in order equals afft_gpu_execute.  (In place, a
+ * single FP32 c / ci of 32768 points is one pass: the range that ends the plan
+ * runs it, others nothing.) */
 int afft_gpu_execute_range(afft_gpu_plan* plan, int first, int last, const void* src_re, const void* src_im,
                            void* dst_re, void* dst_im, void* stream);
 
