@@ -430,8 +430,8 @@ struct Builder {
   // passes ask for wide tiles, whose 4-byte re / im accesses then still cover
   // whole 256-byte row segments)
   //
-  // rows: rows of a plain row pass in one user transform.  Rows of 16384 points
-  // and the r2c of 16384 reals run radix-32 stages in half the LDS (512 and 256
+  // rows: rows of a plain row pass in one user transform (0: radix 16 whatever
+  // their number).  Rows of 16384 points and the r2c of 16384 reals run radix-32 stages in half the LDS (512 and 256
   // threads, two and four groups per CU, so one's loads run beside another's
   // butterflies) once there are more rows than the full-LDS groups of one round
   // on the chip hold.  us, radix-16 / radix-32: c2c 16384 256 rows 18.3 / 23.8,
@@ -535,6 +535,20 @@ struct Builder {
     s.il = 1;
   }
 
+  // Rows of an N-D plan that stay with radix 16 (fft_pass).  With a split side,
+  // radix 16 / 32: c2c 512 x 16384 x 16 1250 / 1314 us, r2c 505 / 538, c2c
+  // 16384^2 3260 / 3394 (1-D rows, which stream, gain in both formats; so does
+  // c2r, 512 x 16384 x 16 852 / 820).  And a c2c whose arrays just fit the 256 MB
+  // MALL, which the column pass then reads again: 512 x 16384 x 4 231 / 261,
+  // 8 x 16384 x 256 261 / 293, 64 x 16384 x 32 219 / 225, 16 x 16 x 16384 x 8
+  // 375 / 391; at 224 MiB and below 0-6 %, from 288 MiB on 1-7 % in favour of
+  // radix 32.
+  bool nd_rows_radix16(const Side& in, const Side& out, idx_t tens) const {
+    if (P.ndim < 2 || P.kind == 3) return false;
+    const idx_t bytes = tens * P.batch * (idx_t)sizeof(cx<T>);
+    return !in.il || !out.il || (P.kind <= 1 && bytes > ((idx_t)224 << 20) && bytes <= ((idx_t)256 << 20));
+  }
+
   // c2c along one axis of the per-user tensor (outer_u, n, inner); in and out
   // carry role/format/offsets and s_u, strides are filled here.
   void axis(Side in, Side out, idx_t outer_u, idx_t n, idx_t inner, int swi, int swo) {
@@ -549,7 +563,7 @@ struct Builder {
     const bool few = inner == 1 && few_points(n * outer_u * P.batch, n >= ((idx_t)1 << 20) ? 22 : 21);
     if (inner == 1 && n <= row_max()) {
       PassRec* r = add();
-      if (!r || !fft_pass(r, (int)n, 0, EPI_PLAIN, 0, 0, outer_u)) return;
+      if (!r || !fft_pass(r, (int)n, 0, EPI_PLAIN, 0, 0, nd_rows_radix16(in, out, tens) ? 0 : outer_u)) return;
       r->in = in;
       r->out = out;
       r->in.s_j = 1;
@@ -700,13 +714,13 @@ struct Builder {
   }
 
   // A single 32768-point transform: one row is one group on one CU, 25.6 us (split
-  // 27.8); as 64 x 512 over 32 and 8 groups 11.0 (12.9).  It keeps the row's independence of
-  // everything but its own buffers (no scratch, so it can be captured at its
-  // first call and run beside any other call): pass A writes the output array,
-  // bin k1 of column j at k1 + 64 j, and pass B works in place there, on the 512
-  // entries k1 + 64 j of row k1, which are also where its bins k1 + 64 k2 go.  A
-  // call in place, where pass A would overwrite input that other groups have
-  // yet to read, runs the row.
+  // 27.8); as 64 x 512 over 32 and 8 groups 11.0 (12.9).  It keeps the row's
+  // independence of everything but its own buffers (no scratch, so it can be
+  // captured at its first call and run beside any other call): pass A writes the
+  // output array, bin k1 of column j at k1 + 64 j, and pass B works in place
+  // there, on the 512 entries k1 + 64 j of row k1, which are also where its bins
+  // k1 + 64 k2 go.  A call in place, where pass A would overwrite input that
+  // other groups have yet to read, runs the row.
   void lone_passes(const Side& in, const Side& out, idx_t n, int swi, int swo) {
     P.in_place = P.pass[--P.npass];
     P.has_in_place = true;
