@@ -45,6 +45,7 @@
 #pragma once
 
 #include "afft_device.h"
+#include "afft_per_device.h"
 
 namespace afgpu {
 
@@ -795,6 +796,17 @@ __device__ __forceinline__ void fft_tile(const PassParams<T>& p, int tile, int t
 template <typename T, int L, int CT, bool COLMAP, bool STORE_T, int SV, bool HX>
 constexpr size_t tile_lds_bytes() {
   return PassShape<L, CT, SV, (!COLMAP && STORE_T) ? (HX ? (int)sizeof(T) : 2 * (int)sizeof(T)) : 0>::template lds_bytes<T, HX>();
+}
+
+// Lets `kernel` be launched with `lds` bytes of dynamic LDS on the current GPU.
+// Above 64 KiB that is an attribute of the function on each device: set once per
+// process, it left a second GPU's launches without it.
+inline hipError_t allow_lds(PerDevice& done, const void* kernel, size_t lds) {
+  if (lds <= 65536) return hipSuccess;
+  int dev = 0;
+  const hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  return done.once(dev, [&] { return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
 }
 
 // Minimum waves per SIMD the compiler must allow for: half-exchange tiles

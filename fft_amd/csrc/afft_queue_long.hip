@@ -180,14 +180,8 @@ __global__ void __launch_bounds__((PassShape<kPairN2, kPairRows>::NT), 4) queue_
 
 template <auto K, typename... Args>
 static hipError_t launch_long(size_t lds, int grid, int threads, hipStream_t st, Args... args) {
-  if (lds > 65536) {
-    static bool attr = false;
-    if (!attr) {
-      hipError_t e = hipFuncSetAttribute((const void*)K, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (e != hipSuccess) return e;
-      attr = true;
-    }
-  }
+  static PerDevice attr;
+  if (hipError_t e = allow_lds(attr, (const void*)K, lds); e != hipSuccess) return e;
   hipLaunchKernelGGL(K, dim3(grid), dim3(threads), lds, st, args...);
   return hipGetLastError();
 }

@@ -528,14 +528,8 @@ template <typename T, int L, int CT, int SV, bool HX>
 static hipError_t launch_r4a(const Real4Args<T>& a, hipStream_t st) {
   using S = R4AShape<T, L, CT, SV, HX>;
   auto k = real4a_kernel<T, L, CT, SV, HX>;
-  if (S::lds > 65536) {
-    static bool attr = false;
-    if (!attr) {
-      hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds);
-      if (e != hipSuccess) return e;
-      attr = true;
-    }
-  }
+  static PerDevice attr;
+  if (hipError_t e = allow_lds(attr, (const void*)k, S::lds); e != hipSuccess) return e;
   const idx_t npc = a.n2 / 2;
   if (npc % CT != 0 || a.n1 != L) return hipErrorInvalidValue;
   const idx_t blocks = a.nbatch * (npc / CT);
@@ -549,14 +543,8 @@ template <typename T, int L, int CT, int SV, bool HX>
 static hipError_t launch_r4b(const Real4Args<T>& a, hipStream_t st) {
   using S = R4BShape<T, L, CT, SV, HX>;
   auto k = real4b_kernel<T, L, CT, SV, HX>;
-  if (S::lds > 65536) {
-    static bool attr = false;
-    if (!attr) {
-      hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds);
-      if (e != hipSuccess) return e;
-      attr = true;
-    }
-  }
+  static PerDevice attr;
+  if (hipError_t e = allow_lds(attr, (const void*)k, S::lds); e != hipSuccess) return e;
   if (a.n2 != L) return hipErrorInvalidValue;
   const idx_t blocks = a.nbatch * ((a.n1 / 2 + 1 + CT - 1) / CT);
   if (blocks <= 0) return hipSuccess;
@@ -569,14 +557,8 @@ template <typename T, int L, int CT, int SV, bool HX>
 static hipError_t launch_r4c(const Real4Args<T>& a, hipStream_t st) {
   using S = R4AShape<T, L, CT, SV, HX>;
   auto k = real4c_kernel<T, L, CT, SV, HX>;
-  if (S::lds > 65536) {
-    static bool attr = false;
-    if (!attr) {
-      hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds);
-      if (e != hipSuccess) return e;
-      attr = true;
-    }
-  }
+  static PerDevice attr;
+  if (hipError_t e = allow_lds(attr, (const void*)k, S::lds); e != hipSuccess) return e;
   if (a.n2 != L || a.rs < a.n1 / 2 + 1) return hipErrorInvalidValue;
   const idx_t blocks = a.nbatch * ((a.n1 / 2 + 1 + CT - 1) / CT);
   if (blocks <= 0) return hipSuccess;
@@ -589,14 +571,8 @@ template <typename T, int L, int CT, int SV, bool HX>
 static hipError_t launch_r4d(const Real4Args<T>& a, hipStream_t st) {
   using S = R4BShape<T, L, CT, SV, HX>;
   auto k = real4d_kernel<T, L, CT, SV, HX>;
-  if (S::lds > 65536) {
-    static bool attr = false;
-    if (!attr) {
-      hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds);
-      if (e != hipSuccess) return e;
-      attr = true;
-    }
-  }
+  static PerDevice attr;
+  if (hipError_t e = allow_lds(attr, (const void*)k, S::lds); e != hipSuccess) return e;
   const idx_t npc = a.n2 / 2;
   if (npc % CT != 0 || a.n1 != L || a.rs < a.n1 / 2 + 1) return hipErrorInvalidValue;
   const idx_t blocks = a.nbatch * (npc / CT);

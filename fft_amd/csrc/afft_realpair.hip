@@ -366,14 +366,8 @@ hipError_t launch_rp(const RealPairArgs<T>& a, idx_t blocks, hipStream_t st) {
   constexpr int SV = 1;
   constexpr size_t lds = rp_lds_bytes<T, L, kRpR, SV>();
   auto k = real_pair_kernel<T, L, kRpR, SV>;
-  if (lds > 65536) {
-    static bool attr = false;
-    if (!attr) {
-      hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (e != hipSuccess) return e;
-      attr = true;
-    }
-  }
+  static PerDevice attr;
+  if (hipError_t e = allow_lds(attr, (const void*)k, lds); e != hipSuccess) return e;
   hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(PassShape<L, 2 * kRpR, SV>::NT), lds, st, a);
   return hipGetLastError();
 }
@@ -401,14 +395,8 @@ static hipError_t launch_rrf(const RealRowFftArgs<T>& a, idx_t blocks, hipStream
   constexpr int SV = 0;
   constexpr size_t lds = PassShape<L, 2, SV>::template lds_bytes<T, true>();
   auto k = real_rowfft_kernel<T, L, SV>;
-  if (lds > 65536) {
-    static bool attr = false;
-    if (!attr) {
-      hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (e != hipSuccess) return e;
-      attr = true;
-    }
-  }
+  static PerDevice attr;
+  if (hipError_t e = allow_lds(attr, (const void*)k, lds); e != hipSuccess) return e;
   hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(PassShape<L, 2, SV>::NT), lds, st, a);
   return hipGetLastError();
 }
@@ -439,14 +427,8 @@ static hipError_t launch_irrf(const RealIRowFftArgs<T>& a, idx_t blocks, hipStre
   constexpr int SV = 0;
   constexpr size_t lds = PassShape<L, 2, SV>::template lds_bytes<T, true>();
   auto k = real_irowfft_kernel<T, L, SV>;
-  if (lds > 65536) {
-    static bool attr = false;
-    if (!attr) {
-      hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (e != hipSuccess) return e;
-      attr = true;
-    }
-  }
+  static PerDevice attr;
+  if (hipError_t e = allow_lds(attr, (const void*)k, lds); e != hipSuccess) return e;
   hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(PassShape<L, 2, SV>::NT), lds, st, a);
   return hipGetLastError();
 }

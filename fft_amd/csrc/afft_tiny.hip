@@ -112,14 +112,8 @@ static hipError_t launch_tiny(const TinyArgs<T>& a, hipStream_t st) {
   constexpr size_t lds = (size_t)R * tiny_pitch<LMAX>() * sizeof(cx<T>);
   static_assert(lds <= 160 * 1024, "LDS of one work-group");
   auto k = tiny_rows_kernel<T, L, EPI, R>;
-  if (lds > 65536) {
-    static bool attr = false;
-    if (!attr) {
-      hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (e != hipSuccess) return e;
-      attr = true;
-    }
-  }
+  static PerDevice attr;
+  if (hipError_t e = allow_lds(attr, (const void*)k, lds); e != hipSuccess) return e;
   if (a.rows <= 0) return hipSuccess;
   const idx_t blocks = (a.rows + R - 1) / R;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
