@@ -45,6 +45,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -368,6 +369,10 @@ struct Queue {
   int* d_counter = nullptr;  // list counters at [l * kCtr], l < kQLists; status at [kStatus * kCtr]
   QListHdr hdr{};
   QListHdr* d_hdr = nullptr;
+  // What every captured launch of this queue can run (its replays run later
+  // lists, but with the kernels and pair groups it was captured with).
+  bool can_rows15 = true, can_rows14 = true;
+  int can_pair_groups = INT_MAX;
   int* d_deps = nullptr;
   size_t cap_deps = 0;
   hipEvent_t done = nullptr;  // recorded after each eager launch; prepare waits for it
@@ -529,11 +534,17 @@ int afft_gpu_queue_prepare(afft_gpu_queue* qh, const afft_gpu_job* jobs, size_t 
     else
       pairs.push_back(i);
   }
-  // few long jobs run as chains, whose tiles spread one job over many CUs
+  // few long jobs run as chains, whose tiles spread one job over many CUs; so do
+  // all where a captured launch lacks a kernel they need
   size_t points = 0;
-  for (size_t i : rows) points += (size_t)1 << (jobs[i].log2n - (jobs[i].kind >= afft_gpu_r ? 1 : 0));
+  bool can = pairs.empty() || q->can_pair_groups > 0;
+  for (size_t i : rows) {
+    const int lgm = jobs[i].log2n - (jobs[i].kind >= afft_gpu_r ? 1 : 0);
+    points += (size_t)1 << lgm;
+    can = can && (lgm == 15 ? q->can_rows15 : q->can_rows14);
+  }
   points += pairs.size() << 16;
-  if (points < (rows.empty() || pairs.empty() ? kLongPoints : kLongPointsMixed)) {
+  if (!can || points < (rows.empty() || pairs.empty() ? kLongPoints : kLongPointsMixed)) {
     big.swap(rows);
     big.insert(big.end(), pairs.begin(), pairs.end());
     pairs.clear();
@@ -563,7 +574,11 @@ int afft_gpu_queue_prepare(afft_gpu_queue* qh, const afft_gpu_job* jobs, size_t 
     scratch_elems += (size_t)1 << lgm;
   }
   const size_t pair_off = scratch_elems;
-  scratch_elems += pairs.size() << 16;
+  if (!pairs.empty()) {
+    // one group at a time, of the fewest groups any launch makes
+    const size_t groups = std::min(queue_pair_groups((int)pairs.size()), q->can_pair_groups);
+    scratch_elems += (pairs.size() + groups - 1) / groups << 16;
+  }
   hipError_t e0 = q_reserve(q->d_scratch, q->cap_scratch, std::max<size_t>(scratch_elems, 1));
   if (e0 != hipSuccess) {
     queue_set_err(hipGetErrorString(e0));
@@ -699,20 +714,25 @@ int afft_gpu_queue_launch(afft_gpu_queue* qh, void* stream) {
   a.status = q->d_counter + kStatus * kCtr;
   a.spin_limit = q->spin_limit;
   a.tab = q->d_tab;
-  // A captured launch runs the lists of whichever prepare is the latest at a
-  // replay, so it takes every kernel this queue's sizes can need; an eager one
-  // leaves out the kernels without a task.
+  // Kernels without a task are left out (an empty one costs a replay 2-3 us).  A
+  // captured launch runs the lists of whichever prepare is the latest at a
+  // replay: it always has the persistent kernel, which can run every job, and
+  // the later prepares keep to what else it has.
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  const bool eager = hipStreamIsCapturing(st, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
-  auto has = [&](int l0, int l1, int lg) {
-    if (eager) return q->hdr.list_off[l0] < q->hdr.list_off[l1];
-    return q->max_lg >= lg && (lg == 0 || q->max_jobs << q->max_lg >= kLongPoints);
-  };
+  const bool known = hipStreamIsCapturing(st, &cs) == hipSuccess;
+  const bool eager = known && cs == hipStreamCaptureStatusNone;
+  auto has = [&](int l0, int l1) { return q->hdr.list_off[l0] < q->hdr.list_off[l1]; };
+  const int npairs = q->hdr.list_off[kQLists] - q->hdr.list_off[QL_PAIR];
+  if (known && !eager) {
+    q->can_rows15 = q->can_rows15 && has(QL_ROW15, QL_ROW14);
+    q->can_rows14 = q->can_rows14 && has(QL_ROW14, QL_PAIR);
+    q->can_pair_groups = std::min(q->can_pair_groups, queue_pair_groups(npairs));
+  }
   hipError_t e = hipSuccess;
-  if (has(QL_ROW15, QL_ROW14, 15)) e = queue_rows(a, QL_ROW15, q->ncu, st);
-  if (e == hipSuccess && has(QL_ROW14, QL_PAIR, 13)) e = queue_rows(a, QL_ROW14, q->ncu, st);
-  if (e == hipSuccess && has(QL_PAIR, kQLists, 16)) e = queue_pairs(a, eager ? q->hdr.list_off[kQLists] - q->hdr.list_off[QL_PAIR] : 0, q->ncu, st);
-  if (e == hipSuccess && has(0, QL_ROW15, 0)) {
+  if (has(QL_ROW15, QL_ROW14)) e = queue_rows(a, QL_ROW15, q->ncu, st);
+  if (e == hipSuccess && has(QL_ROW14, QL_PAIR)) e = queue_rows(a, QL_ROW14, q->ncu, st);
+  if (e == hipSuccess && npairs) e = queue_pairs(a, npairs, st);
+  if (e == hipSuccess && (!eager || has(0, QL_ROW15))) {
     // the full grid even for few tasks: every XCD needs work-groups for its list
     const int grid = q->grid;
     if (q->groups_per_cu == 4)

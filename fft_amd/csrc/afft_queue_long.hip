@@ -14,8 +14,9 @@
 // TB/s), 636 pairs 210 to 270 us (4.9 to 6.3 TB/s over both passes); as chains
 // they took 0.85 ms.  The whole batch: 905 -> 629 us.
 //
-// The launches are persistent under capture (a fixed grid over the prepared
-// lists), so a captured launch runs the lists of the latest prepare.
+// Every kernel reads its list's length on the device and strides over it, so a
+// captured launch runs the lists of the latest prepare on the grid of the one it
+// was captured with.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -131,10 +132,20 @@ __device__ __forceinline__ float* q_pair_scratch(const QArgs& a, int job) {
   return q_global<float>((unsigned long long)(q_const(a.hdr)->pair_scratch + ((idx_t)job << 16)));
 }
 
-__global__ void __launch_bounds__((PassShape<kPairN1, kPairCols>::NT)) queue_pair_a_kernel(QArgs a, int job0, int njobs) {
+// Group `group` of the pair list in `ngroups` equal ones: its first task and its
+// number of jobs (read from the list, so a captured launch splits whichever list
+// is prepared when it is replayed).
+__device__ __forceinline__ void q_pair_group(const QArgs& a, int group, int ngroups, int& off, int& n) {
+  const int all = q_const(a.hdr)->list_off[QL_PAIR + 1] - q_const(a.hdr)->list_off[QL_PAIR];
+  const int per = (all + ngroups - 1) / ngroups;
+  off = q_const(a.hdr)->list_off[QL_PAIR] + group * per;
+  n = min(per, all - group * per);
+}
+
+__global__ void __launch_bounds__((PassShape<kPairN1, kPairCols>::NT)) queue_pair_a_kernel(QArgs a, int group, int ngroups) {
   extern __shared__ __align__(16) unsigned char q_smem[];
-  const int off = q_const(a.hdr)->list_off[QL_PAIR] + job0;
-  const int n = min(njobs, q_const(a.hdr)->list_off[QL_PAIR + 1] - off);
+  int off, n;
+  q_pair_group(a, group, ngroups, off, n);
   constexpr int TILES = kPairN2 / kPairCols;
   for (int i = blockIdx.x; i < n * TILES; i += gridDim.x) {
     const QRec tk = q_rec(a, off + i / TILES);
@@ -154,10 +165,10 @@ __global__ void __launch_bounds__((PassShape<kPairN1, kPairCols>::NT)) queue_pai
   }
 }
 
-__global__ void __launch_bounds__((PassShape<kPairN2, kPairRows>::NT), 4) queue_pair_b_kernel(QArgs a, int job0, int njobs) {
+__global__ void __launch_bounds__((PassShape<kPairN2, kPairRows>::NT), 4) queue_pair_b_kernel(QArgs a, int group, int ngroups) {
   extern __shared__ __align__(16) unsigned char q_smem[];
-  const int off = q_const(a.hdr)->list_off[QL_PAIR] + job0;
-  const int n = min(njobs, q_const(a.hdr)->list_off[QL_PAIR + 1] - off);
+  int off, n;
+  q_pair_group(a, group, ngroups, off, n);
   constexpr int TILES = kPairN1 / kPairRows;
   for (int i = blockIdx.x; i < n * TILES; i += gridDim.x) {
     const QRec tk = q_rec(a, off + i / TILES);
@@ -199,20 +210,17 @@ hipError_t queue_rows(const QArgs& a, int list, int ncu, hipStream_t st) {
 // 676, 668, 629, 629, 664 us; 381 jobs of 6000: 471, 441, 430, 423, 422, 407.
 constexpr int kPairGroup = 448;
 
-hipError_t queue_pairs(const QArgs& a, int njobs, int ncu, hipStream_t st) {
+int queue_pair_groups(int njobs) { return (njobs + kPairGroup - 1) / kPairGroup; }
+
+hipError_t queue_pairs(const QArgs& a, int njobs, hipStream_t st) {
   using SA = PassShape<kPairN1, kPairCols>;
   using SB = PassShape<kPairN2, kPairRows>;
   constexpr size_t la = tile_lds_bytes<float, kPairN1, kPairCols, true, false, 0, false>();
   constexpr size_t lb = tile_lds_bytes<float, kPairN2, kPairRows, false, true, 0, true>();
-  if (njobs == 0) {
-    hipError_t e = launch_long<queue_pair_a_kernel>(la, 4 * ncu, SA::NT, st, a, 0, 0x7fffffff);
-    return e != hipSuccess ? e : launch_long<queue_pair_b_kernel>(lb, 2 * ncu, SB::NT, st, a, 0, 0x7fffffff);
-  }
-  const int groups = (njobs + kPairGroup - 1) / kPairGroup, per = (njobs + groups - 1) / groups;
-  for (int j = 0; j < njobs; j += per) {
-    const int n = std::min(per, njobs - j);
-    hipError_t e = launch_long<queue_pair_a_kernel>(la, n * (kPairN2 / kPairCols), SA::NT, st, a, j, n);
-    if (e == hipSuccess) e = launch_long<queue_pair_b_kernel>(lb, n * (kPairN1 / kPairRows), SB::NT, st, a, j, n);
+  const int groups = queue_pair_groups(njobs), per = (njobs + groups - 1) / groups;
+  for (int g = 0; g < groups; g++) {
+    hipError_t e = launch_long<queue_pair_a_kernel>(la, per * (kPairN2 / kPairCols), SA::NT, st, a, g, groups);
+    if (e == hipSuccess) e = launch_long<queue_pair_b_kernel>(lb, per * (kPairN1 / kPairRows), SB::NT, st, a, g, groups);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

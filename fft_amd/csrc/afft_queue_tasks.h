@@ -48,7 +48,7 @@ struct QTables {
 struct QListHdr {
   int list_off[kQLists + 1];
   int ndeps;  // step counters to clear (4 per chain job)
-  cx<float>* pair_scratch;  // 2^16 entries per pair job, in list order
+  cx<float>* pair_scratch;  // 2^16 entries per job of a pair group
 };
 
 struct QArgs {
@@ -86,8 +86,8 @@ __device__ __forceinline__ QConst<X> q_const(const X* p) {
 // afft_queue_long.hip: the jobs longer than a group tile, without waits
 // between work-groups (each launch follows the previous one on the stream).
 hipError_t queue_rows(const QArgs& a, int list, int ncu, hipStream_t st);
-// njobs > 0: a work-group per tile of that many jobs; 0 (the count is the one
-// prepared when a captured launch is replayed): a fixed grid.
-hipError_t queue_pairs(const QArgs& a, int njobs, int ncu, hipStream_t st);
+// Pass pairs in queue_pair_groups(njobs) groups, njobs = those prepared now.
+int queue_pair_groups(int njobs);
+hipError_t queue_pairs(const QArgs& a, int njobs, hipStream_t st);
 
 }  // namespace afgpu

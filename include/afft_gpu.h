@@ -243,7 +243,11 @@ int afft_gpu_queue_prepare(afft_gpu_queue* q, const afft_gpu_job* jobs, size_t n
  * (the list offsets and counts are read from device memory at run time): a
  * prepare between replays changes what the graph computes, and the caller
  * must let replays finish before calling prepare (prepare only waits for
- * eager launches). */
+ * eager launches).  A captured launch holds the kernels the list prepared at
+ * its capture needs; the one that runs short jobs and chains is always among
+ * them, and later prepares of the queue turn long jobs into chains where a
+ * captured launch lacks the kernel for them: capture with a typical batch
+ * prepared. */
 int afft_gpu_queue_launch(afft_gpu_queue* q, void* stream);
 /* prepare + launch. */
 int afft_gpu_queue_run(afft_gpu_queue* q, const afft_gpu_job* jobs, size_t njobs, void* stream);
