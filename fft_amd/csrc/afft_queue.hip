@@ -820,7 +820,9 @@ int afft_gpu_queue_get_config(const afft_gpu_queue* qh, int* groups_per_cu, int*
 
 // Times every (groups per CU, lag) candidate on this batch -- prepare, one
 // warm launch, `iters` timed launches -- and keeps the fastest whose launches
-// met every dependency; the queue is left prepared with it.
+// met every dependency; the queue is left prepared with it.  A setting that
+// nothing in the batch depends on (the lag without chains, the groups with rows
+// and pairs only) is left as it was: the launches would differ by noise alone.
 int afft_gpu_queue_tune(afft_gpu_queue* qh, const afft_gpu_job* jobs, size_t njobs, void* stream, int iters,
                         float* best_ms) {
   Queue* q = get_queue(qh);
@@ -837,9 +839,13 @@ int afft_gpu_queue_tune(afft_gpu_queue* qh, const afft_gpu_job* jobs, size_t njo
   const int keep_groups = q->groups_per_cu, keep_lag = q->lag;
   float best = 1e30f;
   int bg = keep_groups, bl = keep_lag;
-  bool failed = false;
-  for (int groups : {4, 2}) {
-    for (int lag : {kLag, 32, 8}) {
+  bool failed = afft_gpu_queue_prepare(qh, jobs, njobs) < 0;
+  std::vector<int> try_groups{keep_groups}, try_lags{keep_lag};
+  if (q->hdr.list_off[QL_ROW15] > 0) try_groups = {4, 2};
+  if (q->nchain > 0) try_lags = {kLag, 32, 8};
+  for (int groups : try_groups) {
+    for (int lag : try_lags) {
+      if (failed) break;
       if (afft_gpu_queue_set_groups_per_cu(qh, groups) != 0 || afft_gpu_queue_set_lag(qh, lag) != 0 ||
           afft_gpu_queue_prepare(qh, jobs, njobs) < 0 || afft_gpu_queue_launch(qh, stream) != 0) {
         failed = true;

@@ -273,7 +273,8 @@ int afft_gpu_queue_get_config(const afft_gpu_queue* q, int* groups_per_cu, int* 
 /* Autotuning for a batch (no counterpart in afft, which has no queue): times
  * each (groups per CU, lag) candidate on these jobs -- prepare, one warm
  * launch, `iters` timed launches on `stream` -- keeps the fastest whose
- * launches met every dependency and leaves the queue prepared with it.
+ * launches met every dependency and leaves the queue prepared with it.  A
+ * setting that no job of the batch depends on is not changed.
  * best_ms (optional) receives its time per launch.  The jobs' outputs are
  * written by every candidate (the same values).  Returns 0, or -1. */
 int afft_gpu_queue_tune(afft_gpu_queue* q, const afft_gpu_job* jobs, size_t njobs, void* stream, int iters,
