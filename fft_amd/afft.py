@@ -44,9 +44,10 @@ def required_counts(kind: str, dims, fmt: int, batch: int = 1):
 
 
 def _torch_dtype(dtype):
-    """torch's name of a numpy element type, None while torch is not loaded."""
+    """torch's name of a numpy element type, None while torch is not loaded (by
+    size: the name of a numpy type is built by Python code, 3 us)."""
     t = sys.modules.get("torch")
-    return None if t is None else {"float32": t.float32, "float64": t.float64}[np.dtype(dtype).name]
+    return getattr(t, "float64" if np.dtype(dtype).itemsize == 8 else "float32", None)
 
 
 def addresses(bufs, counts, dtype, tdtype):

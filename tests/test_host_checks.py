@@ -73,3 +73,17 @@ def test_addresses_check_every_call(bad):
     for x in (_FakeDev(bad[0], **bad[1]), None, 0, torch.zeros(128)):
         with pytest.raises(ValueError):
             afft.addresses((_FakeDev(128), None, x, None), cnt, np.float32, t)
+
+
+def test_torch_dtype_runs_no_python_code_of_numpy():
+    import sys
+    calls = []
+    for dt, want in ((np.dtype(np.float32), torch.float32), (np.float32, torch.float32), ("float64", torch.float64),
+                     (np.dtype("float64"), torch.float64)):
+        sys.setprofile(lambda f, ev, arg: calls.append(f.f_code.co_name) if ev == "call" else None)
+        try:
+            got = afft._torch_dtype(dt)
+        finally:
+            sys.setprofile(None)
+        assert got is want
+    assert calls == ["_torch_dtype"] * 4, calls
