@@ -150,7 +150,7 @@ struct Variant {
                       // 1 always, 0 never, 2 (default) unless an N-D plan's arrays fit the MALL
   int xcd_order = 0;  // XCD-contiguous tile order
   idx_t chunk = 0;    // transforms per pass group (0 = default)
-  int sched = 0;      // 1 / 0 (default): radix-32 schedules where compiled, -1: never
+  int sched = 0;      // 1: radix-32 schedules where compiled, -1: never, 0 (default): but for few points or rows
   int half_lds = 0;   // 1 / 0 (default): half-LDS kernels where compiled, -1: never
   int pipeline = 0;   // removed schedule (pass A of group k beside pass B of group k-1): must be <= 0
   int real_pair = 0;  // fused real passes: 1 = all (also 1-D r2c pass B), 0 (default) = the N-D row-pair one, -1 = none
@@ -404,15 +404,17 @@ struct Builder {
   // transform ran 16 and 8 groups, a single 2^20 64 and 128).  Such a four-step
   // takes balanced factors and the narrowest full-LDS radix-16 tiles instead:
   // more, smaller groups, no second exchange.  us, before / after, FP32 c2c:
-  // 2^16 x 1 16.9 / 15.0, 2^17 x 1 19.5 / 14.8, x 4 21.3 / 16.2, 2^18 x 1 20.1 /
-  // 15.5, x 4 24.3 / 20.2, 2^19 x 1 26.1 / 19.0, x 2 30.4 / 22.1, 2^20 x 1 28.7 /
-  // 24.3, x 2 33.4 / 29.4, 2^21 x 1 37 / 32, 2^22 x 1 57.5 / 45.2; 2^20 x 16 and
-  // 2^22 x 2 are faster with the wide tiles.  A variant that names a schedule,
-  // an exchange or a split is followed as it is.
+  // 2^16 x 1 16.0 / 14.0, x 7 17.4 / 15.5, 2^17 x 1 17.3 / 13.4, x 5 20.2 / 16.1,
+  // 2^18 x 1 19.0 / 14.2, x 3 21.9 / 16.8, 2^19 x 1 26.0 / 17.9, x 2 29.2 / 21.4,
+  // 2^20 x 1 28.1 / 23.2, x 2 31.9 / 28.3, 2^21 x 1 36.9 / 30.5, x 2 44.7 / 46.0
+  // (split 95 / 94), 2^22 x 1 53.0 / 43.6; 2^20 x 16 and 2^22 x 2 are faster with
+  // the wide tiles.  A variant that names a tile, a schedule, an exchange, a split
+  // or a real form is followed as it is: a saved one keeps the plan it was tuned
+  // with, and the tuner reaches the wide tiles (sched = 1).
   bool few_points(idx_t points, int lg_limit) const {
     const Variant& v = P.var;
-    return sizeof(T) == 4 && P.mode == afft_gpu_mode_fma && v.sched == 0 && v.half_lds == 0 && v.row_log2 == 0 &&
-           v.fused <= 0 && points <= ((idx_t)1 << lg_limit);
+    return sizeof(T) == 4 && P.mode == afft_gpu_mode_fma && v.col_tile == 0 && v.rowt_tile == 0 && v.sched == 0 &&
+           v.half_lds == 0 && v.row_log2 == 0 && v.real_pair == 0 && v.fused <= 0 && points <= ((idx_t)1 << lg_limit);
   }
 
   // Row length n2 of the 1-D four-step n = n1 * n2: 1024-point rows up to
@@ -970,7 +972,7 @@ struct Builder {
     // 2048-point columns, 16 per group, of a transform or two are fewer groups
     // than CUs: 8 per group (2^22 x 1 56.1 -> 46.4 us, x 2 66.6 -> 62.8, x 4
     // 88.8 -> 97.6; 2^23 x 1 69.1 -> 65.7, x 2 102.9 -> 108.7)
-    const bool narrow = n1 == 2048 && P.var.col_tile == 0 && P.var.real_pair == 0 && P.batch * N <= ((idx_t)1 << 23);
+    const bool narrow = n1 == 2048 && few_points(P.batch * N, 23);
     if (!real4_shape(0, (int)sizeof(T), (int)std::min<idx_t>(n1, 1 << 30), narrow ? 8 : P.var.col_tile, want_sv, want_hx, cta, sva,
                      hxa) ||
         !real4_shape(1, (int)sizeof(T), (int)std::min<idx_t>(n2, 1 << 30), P.var.rowt_tile, want_sv, want_hx, ctb,
@@ -1051,8 +1053,8 @@ struct Builder {
     // the spectrum pass of few points: radix 16 (2^19 x 1 31.4 -> 25.0 us, x 4
     // 30.3 -> 28.5; 2^20 x 1 27.4 -> 26.3, x 4 36.6 -> 34.2; 2^21 x 1 33.6 -> 29.3,
     // x 2 39.4 -> 35.1, x 4 49.7 -> 50.9; 2^22 x 1 39.4 -> 35.8, x 2 50.6 -> 51.8)
-    const bool few = P.var.real_pair == 0 && few_points(N * P.batch, 22);
-    const int col_tile = few && P.var.col_tile == 0 && n2 == 1024 ? 16 : P.var.col_tile;
+    const bool few = few_points(N * P.batch, 22);
+    const int col_tile = few && n2 == 1024 ? 16 : P.var.col_tile;
     if (!real4_shape(2, (int)sizeof(T), (int)std::min<idx_t>(n2, 1 << 30), col_tile, few ? 0 : want_sv,
                      few ? (n2 >= 1024 ? 0 : 1) : want_hx, ctc, svc,
                      hxc) ||
@@ -2558,6 +2560,17 @@ bool tune_impl(Plan& P, const void* sre, const void* sim, void* dre, void* dim, 
     P.var = Variant();
     if (!rebuild<T>(P)) return false;
     base_chunk = P.chunk;
+    // the schedules the default leaves out for few points or rows
+    std::vector<std::tuple<int, int, int, int>> shape[2];
+    for (int sch : {0, 1}) {
+      P.var.sched = sch;
+      if (rebuild<T>(P))
+        for (int i = 0; i < P.npass; i++)
+          shape[sch].emplace_back(P.pass[i].L, P.pass[i].CT, P.pass[i].sv, P.pass[i].hx);
+    }
+    if (!shape[1].empty() && shape[1] != shape[0]) cands.push_back(P.var);
+    P.var = Variant();
+    if (!rebuild<T>(P)) return false;
   }
   // streaming I/O forced on and off, and the XCD-contiguous tile order, on the
   // default shape (each moved N-D transforms by a few per cent either way)

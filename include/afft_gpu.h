@@ -126,8 +126,10 @@ typedef struct
                         non-temporal otherwise */
   int32_t xcd_order; /* 1: hand each XCD a contiguous run of tiles */
   int64_t chunk;     /* transforms per pass group of four-step plans */
-  int32_t sched;     /* 1 or 0 (default): radix-32 stage schedules for the long passes
-                        where compiled, -1: never */
+  int32_t sched;     /* 1: radix-32 stage schedules for the long passes where compiled,
+                        -1: never, 0 (default): as 1 but for few points or rows, where the
+                        plan takes radix-16 tiles that make more work-groups (also only
+                        while no tile, exchange, split or real form is named) */
   int32_t half_lds;  /* 1: half-LDS kernels (real and imaginary parts exchanged in turn)
                         where compiled, -1: never, 0: default (on) */
   int32_t pipeline;  /* must be 0 or -1: the schedule that ran pass A of group k beside
