@@ -59,3 +59,11 @@ def test_named_real_forms(lg):
         for rp in (-1, 1):
             v = dict(real_pair=rp)
             assert _plan(kind, lg, limit, v) == _plan(kind, lg, limit + 1, v), (kind, v)
+
+
+def test_2_20_in_whole_rounds_only():
+    def nd(batch):
+        return [_describe(32, 0, (2, 1 << 20), 1, batch, None, i)[1] for i in range(2)]
+    assert _plan(0, 20, 3) == _plan(0, 20, 5)
+    assert _plan(0, 20, 2) == _plan(0, 20, 4) == _plan(0, 20, 1) != _plan(0, 20, 5)
+    assert " hx " not in nd(1)[1] and " hx " in nd(2)[1], (nd(1), nd(2))
