@@ -1,5 +1,5 @@
-// FP32 instantiations of the pass kernels (row passes here; the _cols and
-// _realcols units include this file for their part).
+// FP32 instantiations of the pass kernels (plain row passes here; the _cols,
+// _realcols and _realrows units include this file for their part).
 // Column tiles: 16 columns (128-byte segments) up to L = 1024; beyond that the
 // 160 KiB LDS of a CU bounds CT * L.
 #ifndef AFGPU_PART

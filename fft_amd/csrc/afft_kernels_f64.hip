@@ -1,6 +1,7 @@
 // FP64 instantiations of the pass kernels (16-byte elements halve what fits
 // in LDS, so tiles are half the FP32 ones and rows stop at 8192, 16384 with
-// half-LDS tiles).
+// half-LDS tiles).  Plain row passes here; the _cols, _realcols and _realrows
+// units include this file for their part.
 #ifndef AFGPU_PART
 #define AFGPU_PART 0
 #endif

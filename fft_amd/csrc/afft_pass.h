@@ -212,8 +212,8 @@ __device__ __forceinline__ void run_stages(Regs<T, L, SV>& v, int t, LdsAt& lat,
           a[r] = cmul(a[r], tp[(r - 1) * NS]);
         });
       } else {
-        // column-mapped: the lanes of a column tile share k, whose R - 1
-        // entries are contiguous
+        // column tiles: lanes share k, whose R - 1 entries are contiguous; and
+        // short rows (above)
         const cx<T>* tp = tw + StageTwOff<L, SV, S>::value + k * (R - 1);
         static_for<R - 1>([&](auto rc) AFGPU_INLINE {
           constexpr int r = decltype(rc)::value + 1;
@@ -806,7 +806,8 @@ inline hipError_t allow_lds(PerDevice& done, const void* kernel, size_t lds) {
   int dev = 0;
   const hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
-  return done.once(dev, [&] { return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
+  return done.once(
+      dev, [&] { return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
 }
 
 // Minimum waves per SIMD the compiler must allow for: half-exchange tiles

@@ -433,14 +433,15 @@ struct Builder {
   // whole 256-byte row segments)
   //
   // rows: rows of a plain row pass in one user transform (0: radix 16 whatever
-  // their number).  Rows of 16384 points and the r2c of 16384 reals run radix-32 stages in half the LDS (512 and 256
-  // threads, two and four groups per CU, so one's loads run beside another's
-  // butterflies) once there are more rows than the full-LDS groups of one round
-  // on the chip hold.  us, radix-16 / radix-32: c2c 16384 256 rows 18.3 / 23.8,
-  // 300 30.5 / 28.5, 2048 135.7 / 132.5; r2c 32768 256 23.2 / 25.1, 300 36.6 /
-  // 28.8, 2048 172 / 142; c2r 32768 256 22.6 / 25.7, 300 35.7 / 33.1, 2048 176
-  // / 167; r2c 16384 512 21.0 / 21.9, 1024 37.2 / 30.8, 4096 139 / 122.  8192
-  // points c2c and c2r lose (114 / 117, 139 / 150) and have no such kernel.
+  // their number).  Rows of 16384 points and the r2c of 16384 reals run radix-32
+  // stages in half the LDS (512 and 256 threads, two and four groups per CU, so
+  // one's loads run beside another's butterflies) once there are more rows than
+  // one round of full-LDS groups holds (one or two rows on each of 256 CUs).  us,
+  // radix-16 / radix-32: c2c 16384 256 rows 18.3 / 23.8, 300 30.5 / 28.5, 2048
+  // 135.7 / 132.5; r2c 32768 256 23.2 / 25.1, 300 36.6 / 28.8, 2048 172 / 142;
+  // c2r 32768 256 22.6 / 25.7, 300 35.7 / 33.1, 2048 176 / 167; r2c 16384 512
+  // 21.0 / 21.9, 1024 37.2 / 30.8, 4096 139 / 122.  8192 points c2c and c2r lose
+  // (114 / 117, 139 / 150) and have no such kernel.
   bool fft_pass(PassRec* r, int L, int colmap, int epi, int store_t, int pref_ct = 0, idx_t rows = 1, bool few = false) {
     // tile: the variant's choice for column / transposed-store passes, else
     // the compiled default; schedule: radix-32 where compiled unless the
@@ -977,8 +978,8 @@ struct Builder {
     // than CUs: 8 per group (2^22 x 1 56.1 -> 46.4 us, x 2 66.6 -> 62.8, x 4
     // 88.8 -> 97.6; 2^23 x 1 69.1 -> 65.7, x 2 102.9 -> 108.7)
     const bool narrow = n1 == 2048 && few_points(P.batch * N, 23);
-    if (!real4_shape(0, (int)sizeof(T), (int)std::min<idx_t>(n1, 1 << 30), narrow ? 8 : P.var.col_tile, want_sv, want_hx, cta, sva,
-                     hxa) ||
+    if (!real4_shape(0, (int)sizeof(T), (int)std::min<idx_t>(n1, 1 << 30), narrow ? 8 : P.var.col_tile, want_sv,
+                     want_hx, cta, sva, hxa) ||
         !real4_shape(1, (int)sizeof(T), (int)std::min<idx_t>(n2, 1 << 30), P.var.rowt_tile, want_sv, want_hx, ctb,
                      svb, hxb) ||
         (n2 / 2) % cta != 0)

@@ -14,12 +14,12 @@
 //   - longer jobs (complex length m = 8192 .. 65536), where they are enough to
 //     fill the GPU, run as whole rows and pass pairs in launches of their own
 //     (afft_queue_long.hip);
-//   - otherwise such a job becomes a chain of tile tasks over its own scratch slot: [real pre-pass tiles (c2r)] -> four-step
-//     pass-A tiles (m/256-point columns, 16..64 columns each, W_m twiddle) ->
-//     pass-B tiles (16 rows of 256 points, columns-fastest store) -> [real
-//     post-pass tiles (r2c)].  Every tile of one step can run on a different
-//     CU; a step waits for the previous step's tiles of the same job through a
-//     per-job counter.
+//   - otherwise such a job becomes a chain of tile tasks over its own scratch
+//     slot: [real pre-pass tiles (c2r)] -> four-step pass-A tiles (m/256-point
+//     columns, 16..64 columns each, W_m twiddle) -> pass-B tiles (16 rows of
+//     256 points, columns-fastest store) -> [real post-pass tiles (r2c)].
+//     Every tile of one step can run on a different CU; a step waits for the
+//     previous step's tiles of the same job through a per-job counter.
 // Placement: each long job is assigned to one of the 8 XCDs (largest first,
 // to the least loaded), and its tiles go to that XCD's task list; a
 // work-group reads its XCD id from the hardware (HW_REG_XCC_ID) and pops its
@@ -75,7 +75,7 @@ constexpr int kLag = 128;        // default jobs between consecutive steps of on
 // 69 / 91, 500 (8 M) 83 / 95, 700 (10.7 M) 125 / 101, 1000 (15 M) 177 / 121;
 // 190 jobs of 2^16 (10.2 M) 114 / 102, 300 (16 M) 176 / 127; 1000 of 2^6..2^16
 // (9 M, both) 104 / 120, 1200 (10.6 M) 126 / 131, 1350 (11.9 M) 137 / 134, 1500
-// (12.9 M) 150 / 138, 3000 283 / 240, 10,000 907 / 604.
+// (12.9 M) 150 / 138, 3000 283 / 240, 10,000 906 / 609.
 constexpr size_t kLongPoints = (size_t)10 << 20, kLongPointsMixed = (size_t)12 << 20;
 constexpr int kStatus = kQLists;  // counter slot of the status flag
 

@@ -9,10 +9,12 @@
 //          a launch over the tiles of a group of such jobs.
 //
 // What bounds them: memory.  Of 10,000 jobs of 2^6..2^16 points (MI355X) 909
-// rows of 2^15 take 184 us (2.6 TB/s: one group per CU, 3.6 rounds of it, loads
-// and butterflies of a row in turn), 1818 rows of 2^13 and 2^14 112 us (3.2
-// TB/s), 636 pairs 210 to 270 us (4.9 to 6.3 TB/s over both passes); as chains
-// they took 0.85 ms.  The whole batch: 905 -> 629 us.
+// rows of 2^15 take 183 us (2.6 TB/s: one group per CU, 3.6 rounds of it, loads
+// and butterflies of a row in turn), 1818 rows of 2^13 and 2^14 111 us (3.2
+// TB/s), 636 pairs 240 us (5.5 TB/s over both passes); as chains they took 0.85
+// ms.  The whole batch: 906 -> 609 us.  With the three kinds of row in one
+// kernel queue_row15_kernel spills 38 VGPRs (132 B a lane), queue_row14_kernel
+// 10; the plans' own kernels of 2^15 points 2 to 14.
 //
 // Every kernel reads its list's length on the device and strides over it, so a
 // captured launch runs the lists of the latest prepare on the grid of the one it
@@ -198,9 +200,10 @@ static hipError_t launch_long(size_t lds, int grid, int threads, hipStream_t st,
 }
 
 hipError_t queue_rows(const QArgs& a, int list, int ncu, hipStream_t st) {
-  if (list == QL_ROW15)
-    return launch_long<queue_row15_kernel>(tile_lds_bytes<float, 32768, 1, false, false, 0, true>(), ncu, 1024, st, a);
-  return launch_long<queue_row14_kernel>(tile_lds_bytes<float, 16384, 1, false, false, 1, true>(), 2 * ncu, 512, st, a);
+  constexpr size_t l15 = tile_lds_bytes<float, 32768, 1, false, false, 0, true>();
+  constexpr size_t l14 = tile_lds_bytes<float, 16384, 1, false, false, 1, true>();
+  if (list == QL_ROW15) return launch_long<queue_row15_kernel>(l15, ncu, 1024, st, a);
+  return launch_long<queue_row14_kernel>(l14, 2 * ncu, 512, st, a);
 }
 
 // Jobs per pass pair: 448 x 512 KiB of scratch, so that pass B still finds most
@@ -220,7 +223,8 @@ hipError_t queue_pairs(const QArgs& a, int njobs, hipStream_t st) {
   const int groups = queue_pair_groups(njobs), per = (njobs + groups - 1) / groups;
   for (int g = 0; g < groups; g++) {
     hipError_t e = launch_long<queue_pair_a_kernel>(la, per * (kPairN2 / kPairCols), SA::NT, st, a, g, groups);
-    if (e == hipSuccess) e = launch_long<queue_pair_b_kernel>(lb, per * (kPairN1 / kPairRows), SB::NT, st, a, g, groups);
+    if (e == hipSuccess)
+      e = launch_long<queue_pair_b_kernel>(lb, per * (kPairN1 / kPairRows), SB::NT, st, a, g, groups);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
